@@ -327,6 +327,72 @@ __global__ __launch_bounds__(256) void quantize_rec_kernel(const float* __restri
     if (o == 0) *reinterpret_cast<float*>(rec + kRecA + (b * 16 + r) * 4) = s;
 }
 
+// Activation records for the INT4 prefill GEMM (kF6Rec): a wave per
+// (16 rows, block); the 4 lanes of a row quantize one block, exchange the
+// base-16 digits of their octets, and lane d packs digit d of the row's 32
+// values (mult = 8: the row's -8 sum(q), or 1: -sum(q)).  Padding rows are
+// zeros.
+template <bool HP>
+__global__ __launch_bounds__(256) void quantize_f6_kernel(const float* __restrict__ A, int M, int K, int nblk,
+                                                          int tiles, int mult, uint8_t* __restrict__ R) {
+    const int g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int o = lane & 3, r = lane >> 2;
+    const int mt = g / nblk, j = g - mt * nblk, m = 16 * mt + r;
+    if (mt >= tiles) return;  // whole waves only: the quad exchanges need all lanes
+    float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f), v1 = v0;
+    if (m < M) {
+        const float* src = A + (size_t)m * K + 32 * j + 8 * o;
+        v0 = *reinterpret_cast<const float4*>(src);
+        v1 = *reinterpret_cast<const float4*>(src + 4);
+    }
+    float s;
+    int sum;
+    uint2 ph, pl;
+    quant4x8<HP>(v0, v1, s, ph, pl, sum);
+    // Digit i of the octet as nibbles in the weights' order (byte b: k = b
+    // low, k = 4 + b high).
+    uint32_t dig[4];
+    auto nibbles = [](uint32_t x, uint32_t y, uint32_t& lo, uint32_t& hi) {
+        lo = (x & 0x0F0F0F0Fu) | ((y & 0x0F0F0F0Fu) << 4);
+        hi = ((x >> 4) & 0x0F0F0F0Fu) | (y & 0xF0F0F0F0u);
+    };
+    if (HP) {
+        nibbles(pl.x ^ 0x80808080u, pl.y ^ 0x80808080u, dig[0], dig[1]);
+        nibbles(ph.x, ph.y, dig[2], dig[3]);
+    } else {
+        nibbles(ph.x, ph.y, dig[0], dig[1]);
+        dig[2] = dig[3] = 0;
+    }
+    // Lane o takes digit o of the quad's four octets.
+    uint32_t w[4], d[6];
+    auto take = [&](auto st) {
+        constexpr int S = decltype(st)::value;
+        uint32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)dig[i], 0x55 * S, 0xF, 0xF, false);
+        w[S] = o & 2 ? (o & 1 ? v[3] : v[2]) : (o & 1 ? v[1] : v[0]);
+    };
+    take(std::integral_constant<int, 0>{});
+    take(std::integral_constant<int, 1>{});
+    take(std::integral_constant<int, 2>{});
+    take(std::integral_constant<int, 3>{});
+    uint32_t ds[6];
+    f6_pack(w, d);
+    f6_pack_signed(w, ds);
+    const bool top = o == (HP ? 3 : 1);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) d[i] = top ? ds[i] : d[i];
+    // Row 4 i + (r & 3)'s scale and sum for lane (r, digit i): from lane 0 of
+    // that row's quad.
+    const int src = 4 * (4 * (4 * o + (r & 3)));
+    const float sr = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(s)));
+    const int sumr = __builtin_amdgcn_ds_bpermute(src, sum);
+    uint8_t* rec = R + ((size_t)mt * nblk + j) * kF6Rec + 16 * (r + 16 * o);
+    *reinterpret_cast<uint4*>(rec) = make_uint4(d[0], d[1], d[2], d[3]);
+    *reinterpret_cast<uint4*>(rec + kF6Plane) =
+        make_uint4(d[4], d[5], __float_as_uint(sr), __float_as_uint((float)(-mult * sumr)));
+}
+
 // Row pairs per prefill workgroup: 32 rows for up to 32 rows, 64 for up to
 // 64, otherwise 128.  `force` (BREEZE_HIP_PREFILL_RP) selects 1, 2 or 4 for
 // tests.
@@ -820,7 +886,11 @@ Scratch* scratch_for(Workspace& w, hipStream_t st) {
 // share the array and race.
 constexpr size_t kNoAllocBytes = 16u << 20;
 constexpr size_t kNoAllocState = 512;
-static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
+// A call's room is counted in the INT8 GEMM's record bytes, so what fits does
+// not depend on the weights' width; the FP6 records of the INT4 GEMM take
+// 4096 / 2176 of that.
+constexpr size_t kNoAllocArray = (kNoAllocBytes / kRecBytes + 1) * 2 * kF6Rec;
+static __device__ __align__(256) uint8_t scratch[kNoAllocArray];
 uint8_t* g_noalloc_ptr[kMaxDevices];
 
 __global__ void fill_u32_kernel(uint32_t* __restrict__ p, int n, uint32_t v) {
@@ -1181,6 +1251,8 @@ constexpr int kPairMaxRows4 = 16;
 constexpr int kDec8LrecTiles = 2;
 constexpr int kPrefillMinRows = 9;
 constexpr int kSplitMaxTiles = 8, kSplitMinPhases = 20;
+constexpr int kPf16TilesPerCu = 13, kPf16DeepPerCu = 6;
+constexpr double kPf4Start = 0.6;
 constexpr int kStreamIdleDiv = 8, kStreamMaxGroups = 2;
 
 // Row-blocks the decode prologue quantizes itself for calls of M rows
@@ -1293,7 +1365,9 @@ struct Plan {
     int RG = 1, NG = 1;      // row groups, tile ranges
     int pair_xcd = 0;        // the row groups of a tile range share an XCD
     int lds = 0;             // dynamic LDS bytes (decode kernels)
-    int pf_rp = 0, pf_ct = 0, Mpad = 0;  // prefill: row pairs, column tiles, padded rows
+    // Prefill: row pairs (0: independent 16-row waves), column tiles, padded
+    // rows, weight chunks in flight of the independent waves.
+    int pf_rp = 0, pf_ct = 0, Mpad = 0, pf_ahead = 0;
     int grid_x = 0, grid_y = 1;
     int split = 0;           // decode split-K: workgroups per tile (0: none)
     bool stream = false;     // decode: weight chunks read with non-temporal loads
@@ -1365,6 +1439,55 @@ int split_pieces(const Shape& h, int M, const CallKind& k, int n_cu, int* lds) {
     return S;
 }
 
+// The INT4 prefill launch (see the routing table): independent 16-row waves up
+// to kPf16TilesPerCu output tiles a CU, else the workgroup shape whose
+// rounds x (half the column groups of a CU's busiest SIMD + kPf4Start) is
+// least; a CU holds eight waves.  BREEZE_HIP_PREFILL_RP / _CT force a workgroup shape,
+// BREEZE_HIP_PF16=0 / 1 turns the independent waves off / on.
+void pick_pf4(Plan& p, int M, int tiles, int n_cu) {
+    const char* frp = std::getenv("BREEZE_HIP_PREFILL_RP");
+    const char* fct = std::getenv("BREEZE_HIP_PREFILL_CT");
+    const char* f16 = std::getenv("BREEZE_HIP_PF16");
+    const long waves = (long)tiles * ((M + 15) / 16);
+    const bool few = waves <= (long)kPf16TilesPerCu * n_cu && !frp && !fct;
+    if (f16 ? f16[0] == '1' : few) {
+        p.pf_rp = 0;
+        p.pf_ct = 1;
+        p.pf_ahead = waves <= (long)kPf16DeepPerCu * n_cu ? 4 : 2;
+        p.grid_x = (int)((waves + 3) / 4);
+        p.grid_y = 1;
+        return;
+    }
+    const int rp = frp ? std::atoi(frp) : 0, ct = fct ? std::atoi(fct) : 0;
+    bool rp_ok = false, ct_ok = false;
+    for (const PfCfg& c : kPfCfgs) {
+        rp_ok = rp_ok || c.rp == rp;
+        ct_ok = ct_ok || ((!rp || c.rp == rp) && c.ct == ct);
+    }
+    double best = -1.0;
+    for (const PfCfg& c : kPfCfgs) {
+        if ((rp_ok && c.rp != rp) || (ct_ok && c.ct != ct)) continue;
+        const int groups = (c.ct + 1) / 2, parts = std::min(groups, kPfWaves / c.rp), waves_wg = c.rp * parts;
+        const int per_cu = std::max(1, kPfWaves / waves_wg);
+        int simd = 0;  // column groups on the busiest SIMD of a CU
+        for (int sm = 0; sm < 4; ++sm) {
+            int n = 0;
+            for (int w = sm; w < waves_wg; w += 4) n += groups / parts + (w / c.rp < groups % parts);
+            simd = std::max(simd, n * per_cu);
+        }
+        const long gx = (tiles + c.ct - 1) / c.ct, gy = (M + 32 * c.rp - 1) / (32 * c.rp);
+        const long slots = (long)n_cu * per_cu;
+        const double cost = (double)((gx * gy + slots - 1) / slots) * (0.5 * simd + kPf4Start);
+        if (best < 0 || cost < best || (cost == best && c.rp == 2 && c.ct == 8)) {
+            best = cost;
+            p.pf_rp = c.rp;
+            p.pf_ct = c.ct;
+            p.grid_x = (int)gx;
+            p.grid_y = (int)gy;
+        }
+    }
+}
+
 Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
     Plan p;
     const int JG = h.bits == 8 ? 2 : 4;
@@ -1425,6 +1548,10 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
         const int rows = 32 * p.pf_rp;
         p.Mpad = (M + rows - 1) / rows * rows;
         p.grid_y = p.Mpad / rows;
+        if (h.bits == 4) {
+            pick_pf4(p, M, tiles, n_cu);
+            return p;
+        }
         p.pf_ct = pick_pf_ct(tiles, p.grid_y, p.pf_rp, n_cu, std::getenv("BREEZE_HIP_PREFILL_CT"));
         p.grid_x = (tiles + p.pf_ct - 1) / p.pf_ct;
     } else if (dec8) {
@@ -1551,12 +1678,24 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
     if (p.quant == kQuantPrefill) {
         // Records in MFMA operand order for the prefill GEMM.
         const int nch_rec = (h->nblk + 1) / 2;  // record chunks of two blocks
-        if (!grow(w, st, &s.rec, &s.rec_cap, (size_t)(p.Mpad / 16) * nch_rec * kRecBytes, "workspace alloc", s.fixed))
-            return -4;
-        const size_t threads = (size_t)(p.Mpad / 16) * nch_rec * 2 * 64;  // a wave per (16 rows, block)
-        const unsigned qb = (unsigned)((threads + 255) / 256);
-        if (hp) quantize_rec_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, p.Mpad, s.rec);
-        else quantize_rec_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, p.Mpad, s.rec);
+        const size_t int8_bytes = (size_t)(p.Mpad / 16) * nch_rec * kRecBytes;
+        if (h->bits == 4) {
+            const int rtiles = (M + 31) / 32 * 2, mult = h->Z ? 1 : 8;
+            // The fixed scratch counts the INT8 records' bytes (the array is
+            // larger by the FP6 records' share, kNoAllocArray).
+            const size_t bytes = s.fixed ? int8_bytes : (size_t)rtiles * h->nblk * kF6Rec;
+            if (!grow(w, st, &s.rec, &s.rec_cap, bytes, "workspace alloc", s.fixed)) return -4;
+            const size_t waves = (size_t)rtiles * h->nblk;  // a wave per (16 rows, block)
+            const unsigned qb = (unsigned)((waves + 3) / 4);
+            if (hp) quantize_f6_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, rtiles, mult, s.rec);
+            else quantize_f6_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, rtiles, mult, s.rec);
+        } else {
+            if (!grow(w, st, &s.rec, &s.rec_cap, int8_bytes, "workspace alloc", s.fixed)) return -4;
+            const size_t threads = (size_t)(p.Mpad / 16) * nch_rec * 2 * 64;  // a wave per (16 rows, block)
+            const unsigned qb = (unsigned)((threads + 255) / 256);
+            if (hp) quantize_rec_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, p.Mpad, s.rec);
+            else quantize_rec_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, p.Mpad, s.rec);
+        }
         if (!hip_ok(hipGetLastError(), "quantize launch")) return -5;
     } else if (p.quant == kQuantRows8) {
         const int rows8 = dec8_rows(M);
@@ -1714,33 +1853,54 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
         else e = hp ? launch_dec_bits<4, true>(w.attr_set, a, p.grid_x, p.lds, fz, p64, fu, x, st)
                     : launch_dec_bits<4, false>(w.attr_set, a, p.grid_x, p.lds, fz, p64, fu, x, st);
     } else if (p.route == kRoutePrefill) {
-        PfArgs pa{};
-        pa.W = reinterpret_cast<const char*>(h->W);
-        pa.WS = reinterpret_cast<const char*>(h->WS);
-        pa.S = reinterpret_cast<const char*>(h->S);
-        pa.Z = reinterpret_cast<const char*>(h->Z);
-        pa.R = reinterpret_cast<const char*>(s.rec);
-        pa.C = dC;
-        pa.M = M;
-        pa.N = h->N;
-        pa.nblk = h->nblk;
-        pa.nch = (h->nblk + 1) / 2;
-        pa.ngrp = h->ngrp;
-        pa.sc_shift = h->sc_shift;
-        pa.ntiles = h->N / 16;
-        pa.nbg = h->nbg;
-        const int scm = h->sc_blk ? 2 : (h->sc_shift == 31 ? 0 : 1);
-        if (h->bits == 4 && scm == 2 && !h->Z) {
-            set_err("internal: INT4 handle with per-block scales has no zero points");
-            return -5;
-        }
         const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y);
-        if (h->bits == 8)
-            e = hp ? launch_pf<8, true>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st)
-                   : launch_pf<8, false>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st);
-        else
-            e = hp ? launch_pf<4, true>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st)
-                   : launch_pf<4, false>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st);
+        if (h->bits == 4) {
+            Pf4Args pa{};
+            pa.W = reinterpret_cast<const char*>(h->W);
+            pa.S = reinterpret_cast<const char*>(h->S);
+            pa.Z = reinterpret_cast<const char*>(h->Z);
+            pa.R = reinterpret_cast<const char*>(s.rec);
+            pa.C = dC;
+            pa.M = M;
+            pa.N = h->N;
+            pa.nblk = h->nblk;
+            pa.nbg = h->nbg;
+            pa.ntiles = h->N / 16;
+            if (h->sc_blk) {  // [tile][chunk][16][4]
+                pa.sc_shift = 2;
+                pa.s_tile = (size_t)h->nbg * 256;
+                pa.s_grp = 256;
+                pa.s_col = 16;
+                pa.s_blk = 4;
+            } else {  // [tile][group][16]
+                pa.sc_shift = h->sc_shift;
+                pa.s_tile = (size_t)h->ngrp * 64;
+                pa.s_grp = 64;
+                pa.s_col = 4;
+                pa.s_blk = 0;
+            }
+            const bool zp = h->Z != nullptr;
+            if (p.pf_rp == 0) e = launch_pf16(pa, zp, p.pf_ahead, p.grid_x, st);
+            else e = hp ? launch_pf4<true>(w.pf_attr, pa, zp, p.pf_rp, p.pf_ct, grid, st)
+                        : launch_pf4<false>(w.pf_attr, pa, zp, p.pf_rp, p.pf_ct, grid, st);
+        } else {
+            PfArgs pa{};
+            pa.W = reinterpret_cast<const char*>(h->W);
+            pa.WS = reinterpret_cast<const char*>(h->WS);
+            pa.S = reinterpret_cast<const char*>(h->S);
+            pa.R = reinterpret_cast<const char*>(s.rec);
+            pa.C = dC;
+            pa.M = M;
+            pa.N = h->N;
+            pa.nblk = h->nblk;
+            pa.nch = (h->nblk + 1) / 2;
+            pa.ngrp = h->ngrp;
+            pa.sc_shift = h->sc_shift;
+            pa.ntiles = h->N / 16;
+            const int scm = h->sc_blk ? 2 : (h->sc_shift == 31 ? 0 : 1);
+            e = hp ? launch_pf<true>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st)
+                   : launch_pf<false>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st);
+        }
     } else {
         const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y);
         if (h->bits == 8) e = hp ? launch_rows_bits<8, true>(a, grid, dots, st)
@@ -2141,7 +2301,7 @@ int i4_matmul_noalloc_dev(void* handle, const float* dA, int M, float* dC, int64
     s.fixed = true;
     s.stream = st;
     s.ticket = reinterpret_cast<unsigned int*>(base);
-    s.parts = reinterpret_cast<unsigned long long*>(base + kNoAllocBytes - parts_bytes);
+    s.parts = reinterpret_cast<unsigned long long*>(base + kNoAllocArray / 256 * 256 - parts_bytes);
     s.parts_cap = parts_bytes / sizeof(unsigned long long);
     uint8_t* recs = base + kNoAllocState;
     s.rec = recs;

@@ -599,15 +599,6 @@ constexpr int kLdsMax = 160 * 1024;
 // compiler does not see these loads: every
 // wave waits for its own with an explicit vmcnt, then the workgroup barrier
 // publishes the stage.
-//
-// INT4 weights (BITS 4) take the same core.  A stage is one INT4 chunk (four
-// blocks, 1 KB per tile), loaded raw into chunk 0's weight area; its scales
-// and zero points go to one raw area shared by both stages.  After the
-// stage barrier all 512 threads expand it in place: per byte, b = nibble -
-// zp as a signed byte (n + (128 - zp)) ^ 0x80, chunk 0 getting blocks 0-1
-// and chunk 1 blocks 2-3 in the INT8 chunk layout, plus 128 * sum(b) per
-// (column, block) for the two-pass product and the scales in the INT8
-// chunk layout.  A second barrier publishes the expanded stage.
 
 constexpr int kPfWaves = 8;
 // Chunks per ring stage.
@@ -621,61 +612,41 @@ constexpr int kRecA = 2048, kRecBytes = kRecA + 128;
 // Byte of (row r, k-octet o) in a block's h half of a record.
 __host__ __device__ constexpr int pf_rec_byte(int r, int o) { return 16 * (r + 16 * (o >> 1)) + 8 * (o & 1); }
 // Byte of (column c, k-octet o) of block b in a weight tile's 1 KB in LDS.
-// INT8 tiles arrive by DMA in the decode chunk order (octet o of both blocks
-// at 16 (c + 16 o)), so a 32x32x32 B operand takes two 8-byte halves.  INT4
-// tiles are expanded in LDS into [column half][k half][block][column c & 7]
-// [16 B]: one conflict-free 16-byte read per operand.
-__host__ __device__ constexpr int pf_w_byte(int bits, int c, int o, int b) {
-    return bits == 8 ? 16 * (c + 16 * o) + 8 * b : 16 * ((c & 7) + 8 * b + 16 * (o >> 1) + 32 * (c >> 3)) + 8 * (o & 1);
-}
+// Tiles arrive by DMA in the decode chunk order (octet o of both blocks at
+// 16 (c + 16 o)), so a 32x32x32 B operand takes two 8-byte halves.
+__host__ __device__ constexpr int pf_w_byte(int c, int o, int b) { return 16 * (c + 16 * o) + 8 * b; }
 
 struct PfArgs {
-    const char* W;   // INT8: [ntiles][nch][64 lanes][16 B]; INT4: [ntiles][nbg][64][16 B]
-    const char* WS;  // INT8: [ntiles][nch][16][2] int32
+    const char* W;   // [ntiles][nch][64 lanes][16 B]
+    const char* WS;  // [ntiles][nch][16][2] int32
     const char* S;   // scales (grp_index / blk_index layouts)
-    const char* Z;   // INT4 per-block zero points [ntiles][nbg][16][4] (SCM 2 only)
     const char* R;   // activation records [Mpad/16][nch][kRecBytes]
     float* C;        // [M][N]
     int M, N, nblk, nch, ngrp, sc_shift, ntiles;
-    int nbg;         // INT4: 4-block chunks per tile
 };
 
 // SCM: scale layout: 0 one per column, 1 per group of >= 2 blocks, 2 per block.
 // One chunk's LDS region: [CT weight tiles, 1 KB each][weight sums, 128 B
-// per tile][block or group scales][2 RP activation records].  INT4 adds kNRaw
-// raw areas after the S stages, stage g using area g % kNRaw: S - 1 when a
-// barrier follows the expansion (only the next stage waits for its expansion
-// while the one after it loads), S with one row pair, whose waves expand
-// their own tiles with no barrier after it (a wave may load stage g + S - 1
-// while another still expands stage g).  A raw area holds group scales
-// (SCM 1, 64 B per tile) or block scales then zero points (SCM 2, 256 + 64 B
-// per tile), in whole KB.
-template <int CT, int SCM, int BITS, int RP, int S>
+// per tile][block or group scales][2 RP activation records].
+template <int CT, int SCM, int RP, int S>
 struct PfLayout {
     static constexpr int kWS = CT * 1024;
     static constexpr int kSB = kWS + CT * 128;
     static constexpr int kSharedUsed = kSB + (SCM == 2 ? CT * 128 : SCM == 1 ? CT * 64 : 0);
-    // INT8 pads the sums and scales to whole KB: their 1 KB loads start
+    // The sums and scales are padded to whole KB: their 1 KB loads start
     // where the weight tiles end and must not run into the records.
-    static constexpr int kShared = BITS == 8 ? kWS + (kSharedUsed - kWS + 1023) / 1024 * 1024 : kSharedUsed;
+    static constexpr int kShared = kWS + (kSharedUsed - kWS + 1023) / 1024 * 1024;
     static constexpr int kA = kShared;
     static constexpr int kChunk = kA + 2 * RP * kRecBytes;
     static constexpr int kStage = kPfChunks * kChunk;
-    static constexpr int kRawZ = CT * 256;  // SCM 2: zero points after the block scales
-    static constexpr int kRawUsed = BITS == 8 ? 0 : SCM == 2 ? CT * 320 : SCM == 1 ? CT * 64 : 0;
-    static constexpr int kRaw = (kRawUsed + 1023) / 1024 * 1024;
-    static constexpr int kRawOff = S * kStage;  // raw area r at kRawOff + r * kRaw
-    static constexpr int kNRaw = RP == 1 ? S : S - 1;
-    // INT8, per chunk: CT weight tiles of 1 KB, kWJ a wave; then the sums
-    // and scales in kSU units of 1 KB, kSJ a wave.
-    static constexpr int kWJ = BITS == 8 ? (CT + kPfWaves - 1) / kPfWaves : 0;
-    static constexpr int kSU = BITS == 8 ? (kShared - kWS) / 1024 : 0;
+    // Per chunk: CT weight tiles of 1 KB, kWJ a wave; then the sums and
+    // scales in kSU units of 1 KB, kSJ a wave.
+    static constexpr int kWJ = (CT + kPfWaves - 1) / kPfWaves;
+    static constexpr int kSU = (kShared - kWS) / 1024;
     static constexpr int kSJ = (kSU + kPfWaves - 1) / kPfWaves;
-    // INT4, per stage: the CT raw tiles and the raw area in units of 1 KB.
-    static constexpr int kUnits = CT + kRaw / 1024;
-    // Shared loads a wave issues per chunk (INT8) or stage (INT4).
-    static constexpr int kPerWave = BITS == 8 ? kWJ + kSJ : (kUnits + kPfWaves - 1) / kPfWaves;
-    static constexpr int kBytes = kRawOff + kNRaw * kRaw;
+    // Shared loads a wave issues per chunk.
+    static constexpr int kPerWave = kWJ + kSJ;
+    static constexpr int kBytes = S * kStage;
     static_assert(kShared % 64 == 0 && kBytes <= 160 * 1024, "layout");
 };
 
@@ -706,6 +677,160 @@ struct PfCfg {
 constexpr PfCfg kPfCfgs[] = {{4, 17, 2}, {4, 16, 2}, {4, 13, 2}, {4, 12, 2}, {4, 9, 2}, {4, 8, 2}, {4, 5, 2},
                              {4, 4, 2},  {2, 16, 2}, {2, 8, 3},  {2, 4, 3},  {1, 16, 2}, {1, 8, 3}};
 constexpr int kPfNumCfgs = sizeof(kPfCfgs) / sizeof(kPfCfgs[0]);
+
+// ------------------------------------------------------------------ INT4 prefill on FP6 matrix instructions
+//
+// q (INT16) is four base-16 digits, q = sum d_i 16^i with d_0..d_2 in 0..15
+// and d_3 in -8..7 (INT8 activations: two digits, d_1 in -8..7), and a weight
+// is its nibble n in 0..15.  Both are FP6 E2M3 values times 8: the code of an
+// integer up to 16 in magnitude is its sign and its binary magnitude.  One
+// v_mfma_scale_f32_32x32x64_f8f6f4 multiplies two digits of 32 rows with one
+// block of 32 columns (lanes 0-31 hold the even digit, lanes 32-63 the odd
+// one, and both halves the same weights); the block scales give the digits
+// their powers of 16.  Every partial sum of
+//   P = sum q n,  and of  P - 8 sum(q) = cs for the default zero point,
+// is an integer below 15.8 M < 2^24 in any order, so the FP32 result is exact:
+// the epilogue needs no integer conversion and no weight sums, a multiply and
+// an FMA per (row, column, block) against four instructions on INT8 MFMAs.
+// Explicit zero points take cs = fma(z, -sum(q), P), one correctly rounded
+// step from the exact integer, as the conversion of the integer is.
+
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// Activation record per (16 rows, block), 2 KB: two planes of 64 lanes x 16 B,
+// lane r + 16 i for digit i of row r.  Plane 0: dwords 0-3 of the 32 codes;
+// plane 1: dwords 4-5, then the block scale and -sum(q) (times 8 without
+// explicit zero points) of row 4 i + (r & 3), the row of result r & 3 of lane
+// r + 16 i of v_mfma_scale_f32_16x16x128_f8f6f4.
+constexpr int kF6Plane = 1024, kF6Rec = 2 * kF6Plane;
+
+// 32 nibbles (four octets in the decode chunk order) as 32 six-bit fields, in
+// an order that takes few shifts: weights and activation digits go through
+// the same packing, so the order of k cancels.  Per octet pair, the nibbles of
+// a and b that sit a multiple of 12 bits apart are fields already one, or
+// two bits left of, their place.
+__host__ __device__ inline void f6_pack(const uint32_t* w, uint32_t* d) {
+    for (int p = 0; p < 2; ++p) {
+        const uint32_t a = w[2 * p], b = w[2 * p + 1], t = b << 2;
+        d[3 * p] = (a & 0x0F00F00Fu) | ((a << 2) & 0xC03C03C0u);
+        d[3 * p + 1] = (b & 0xF00F00F0u) | (t & 0x03C03C00u) | (a >> 30);
+        d[3 * p + 2] = (t & 0x3C03C03Cu) | (a & 0x00F00F00u);
+    }
+}
+// A chunk's 16 bytes of lane (column c, octet o) are that octet of four blocks;
+// afterwards lane (c, j) holds the four octets of block j (a 4x4 transpose
+// over the lane quarters).  One 16-byte load and four lane swaps: four 4-byte
+// loads of the same bytes took four times the vector memory issue, which
+// bounds the shapes with few rows.
+__device__ inline void octets_of_block(const uint4& r, uint32_t* w) {
+    const auto a = __builtin_amdgcn_permlane32_swap(r.x, r.z, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(r.y, r.w, false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    w[0] = c[0];
+    w[1] = c[1];
+    w[2] = d[0];
+    w[3] = d[1];
+}
+// The same for signed nibbles (two's complement, -8..7): sign and magnitude.
+__host__ __device__ inline void f6_pack_signed(const uint32_t* w, uint32_t* d) {
+    uint32_t mag[4], sgn[4], e[6];
+    for (int o = 0; o < 4; ++o) {
+        const uint32_t s = (w[o] >> 3) & 0x11111111u;
+        mag[o] = (w[o] ^ (s * 15u)) + s;  // at most 8: no carry between nibbles
+        sgn[o] = s << 3;
+    }
+    f6_pack(mag, d);
+    f6_pack(sgn, e);  // bit 3 of each field; the sign is bit 5
+    for (int i = 0; i < 6; ++i) d[i] |= (e[i] << 2) | (i ? e[i - 1] >> 30 : 0u);
+}
+
+__device__ inline v16f mfma_f6(const v8i& a, const v8i& b, const v16f& c, int sa, int sb) {
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 2, 0, sa, 0, sb);
+}
+
+// The same for one block of 16 rows by 16 columns, all four digits (a lane's
+// 32 k of digit l >> 4).
+__device__ inline v4f mfma_f6_16(const v8i& a, const v8i& b, const v4f& c, int sa, int sb) {
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 2, 0, sa, 0, sb);
+}
+
+// Lane J of each 16-lane row, in every lane of the row.
+template <int J>
+__device__ inline float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + J, 0xF, 0xF, true));
+}
+
+// acc[i] = fma(lane i of the 16-lane row's s, f[i], acc[i]) for i < 4; see
+// fma_rows8.
+__device__ inline void fma_rows4(v4f& acc, float s, const v4f& f) {
+    float a0 = acc[0], a1 = acc[1], a2 = acc[2], a3 = acc[3];
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %4, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %4, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %4, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf"
+        : "+&v"(a0), "+&v"(a1), "+&v"(a2), "+&v"(a3)
+        : "v"(s), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]));
+    acc = v4f{a0, a1, a2, a3};
+}
+
+// acc[i] = fma(lane J0 + i of the 16-lane row's s, f[i], acc[i]) for i < 8, as
+// eight v_fmac_f32 with the row broadcast as a DPP operand.  The s_nop covers
+// the two wait states a DPP read needs after a vector write of s.
+template <int J0>
+__device__ inline void fma_rows8(float* acc, float s, const float* f) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %8, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %8, %10 row_newbcast:%18 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %8, %11 row_newbcast:%19 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %8, %12 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %4, %8, %13 row_newbcast:%21 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %5, %8, %14 row_newbcast:%22 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %6, %8, %15 row_newbcast:%23 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %7, %8, %16 row_newbcast:%24 row_mask:0xf bank_mask:0xf"
+        : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]), "+&v"(acc[5]), "+&v"(acc[6]),
+          "+&v"(acc[7])
+        : "v"(s), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(f[4]), "v"(f[5]), "v"(f[6]), "v"(f[7]), "n"(J0),
+          "n"(J0 + 1), "n"(J0 + 2), "n"(J0 + 3), "n"(J0 + 4), "n"(J0 + 5), "n"(J0 + 6), "n"(J0 + 7));
+}
+
+// A uniform byte offset the optimizer cannot fold into per-lane addresses.
+__device__ inline uint32_t uniform_offset(uint32_t x) {
+    x = (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+    asm("" : "+s"(x));
+    return x;
+}
+
+struct Pf4Args {
+    const char* W;  // [ntiles][nbg][64 lanes][16 B]
+    const char* S;  // scales: of (tile t, column c, block j) at t s_tile + (4 (j / 4) >> sc_shift) s_grp + c s_col + (j & 3) s_blk
+    const char* Z;  // per-block zero points [ntiles][nbg][16][4], or NULL (8 everywhere)
+    const char* R;  // activation records [16-row tiles][nblk]
+    float* C;       // [M][N]
+    int M, N, nblk, nbg, ntiles, sc_shift;
+    int s_grp, s_col, s_blk;
+    size_t s_tile;
+};
+
+// A workgroup of RP row pairs (32 rows each) by CT column tiles: groups of two
+// tiles (32 columns) split over kParts waves per row pair.
+template <int CT, int RP>
+struct Pf4Shape {
+    static constexpr int kGroups = (CT + 1) / 2;
+    static constexpr int kParts = kGroups < 8 / RP ? kGroups : 8 / RP;
+    static constexpr int kGroupBase = kGroups / kParts, kGroupRem = kGroups % kParts;
+    static constexpr int kWaves = RP * kParts;
+    static constexpr int kThreads = 64 * kWaves;
+    // LDS of one stage (four blocks): per group and block 32 columns x 32 B
+    // (the operand, the scale, the zero point), then per block and row pair
+    // the 32 row scales and 32 sums; two stages.
+    static constexpr int kMeta = kGroups * 4096;
+    static constexpr int kStage = kMeta + 4 * RP * 256;
+    static_assert(CT / kWaves <= 4 && 2 * kStage <= 160 * 1024, "shape");
+};
 
 // ------------------------------------------------------------------ decode in row groups of eight
 //
@@ -754,7 +879,10 @@ hipError_t launch_dec_bits(bool* attr_set, const GemvArgs& a, int grid, int lds,
 template <int BITS, bool HP>
 hipError_t launch_dec8(bool* attr_set, const GemvArgs& a, const uint4* rec, int grid, int lds, int fuse, bool extra,
                        bool lrec, hipStream_t st);
-template <int BITS, bool HP>
+template <bool HP>
 hipError_t launch_pf(bool* pf_attr, const PfArgs& p, int scm, int rp, int ct, dim3 grid, hipStream_t st);
+hipError_t launch_pf16(const Pf4Args& p, bool zp, int ahead, int grid, hipStream_t st);
+template <bool HP>
+hipError_t launch_pf4(bool* pf_attr, const Pf4Args& p, bool zp, int rp, int ct, dim3 grid, hipStream_t st);
 
 }  // namespace bq

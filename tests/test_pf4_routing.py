@@ -1,0 +1,47 @@
+"""Which launch an INT4 prefill call takes (pick_pf4 in csrc/qmm.hip): few
+output tiles a CU go to independent 16-row waves (pf_rp 0), more to the
+workgroup shape with the fewest rounds of column groups."""
+import pytest
+
+TABLE = [
+    # (M, K, N) -> plan fields
+    ((33, 5120, 5120), dict(pf_rp=0, grid_x=240, grid_y=1)),
+    ((64, 17408, 5120), dict(pf_rp=0, grid_x=320)),
+    ((166, 4096, 4096), dict(pf_rp=0, grid_x=704)),   # 11 tiles a CU
+    ((256, 4096, 4096), dict(pf_rp=2, pf_ct=8)),      # 16
+    ((64, 5120, 17408), dict(pf_rp=2, pf_ct=8, grid_x=136, grid_y=1)),
+    ((200, 5120, 17408), dict(pf_rp=4, pf_ct=9, grid_x=121, grid_y=2)),
+    ((512, 5120, 17408), dict(pf_rp=4, pf_ct=17, grid_x=64, grid_y=4)),
+]
+
+
+@pytest.mark.parametrize("shape,want", TABLE, ids=[str(t[0]) for t in TABLE])
+def test_int4_prefill_launch(hb, shape, want):
+    M, K, N = shape
+    got = hb.plan(4, M, K, N, n_cu=256)
+    assert got["route"] == "prefill"
+    assert {k: got[k] for k in want} == want, got
+
+
+def test_overrides(hb, monkeypatch):
+    monkeypatch.setenv("BREEZE_HIP_PF16", "0")
+    assert hb.plan(4, 33, 5120, 5120)["pf_rp"] != 0
+    monkeypatch.setenv("BREEZE_HIP_PF16", "1")
+    assert hb.plan(4, 512, 5120, 17408)["pf_rp"] == 0
+    monkeypatch.delenv("BREEZE_HIP_PF16")
+    monkeypatch.setenv("BREEZE_HIP_PREFILL_RP", "2")
+    monkeypatch.setenv("BREEZE_HIP_PREFILL_CT", "16")
+    p = hb.plan(4, 33, 5120, 5120)
+    assert (p["pf_rp"], p["pf_ct"]) == (2, 16)
+
+
+@pytest.mark.parametrize("M", [33, 64, 100, 128, 256, 512, 1000, 4096])
+@pytest.mark.parametrize("N", [16, 48, 1024, 5120, 17408, 151936])
+def test_every_output_is_covered(hb, M, N):
+    p = hb.plan(4, M, 5120, N)
+    if p["route"] != "prefill":
+        return
+    if p["pf_rp"] == 0:
+        assert p["grid_x"] * 4 >= N // 16 * -(-M // 16)
+    else:
+        assert p["grid_x"] * p["pf_ct"] >= N // 16 and p["grid_y"] * 32 * p["pf_rp"] >= M

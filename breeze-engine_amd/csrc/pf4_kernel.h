@@ -6,6 +6,26 @@
 
 namespace bq {
 
+// Bound: VALU and MFMA issue.  A step (a block's 32 rows by 32 columns) is two
+// matrix instructions (18 ns each on one SIMD) and 32 vector instructions
+// (24 ns with two waves issuing); on this GPU the two overlap little, and a
+// copy of the compute alone takes 74-85 ns a step whatever the order of its
+// instructions, 120 us at K=5120 N=17408 and 512 rows.  The kernel takes 153
+// there: operand loads (vector memory issue, 16 cycles of the CU per 1 KB
+// load) and the expansion of the weights add the rest.  On INT8 matrix
+// instructions (64 vector instructions a step) it took 196.
+//
+// Split: wave (rp, part) takes 32 rows and its part of the workgroup's column
+// groups.  The rows' operands go from L2 straight to registers, reused over
+// the wave's groups (through LDS they would cost as much as the weights do);
+// weights are expanded once a workgroup, through LDS, a stage (four blocks)
+// ahead.  Every load has a stage to land: loads complete in order, so a short
+// prefetch of the rows would wait for the weights' latency (163 us against
+// 176 with the rows one block ahead).
+//
+// The row scale enters as a DPP operand (fma_rows8): one register instead of
+// 16 a block.
+
 // One block's A operands of a wave (32 rows): the base-16 digits of q, two
 // digits a matrix instruction.
 template <bool HP>
@@ -313,7 +333,6 @@ hipError_t launch_pf4_zp(bool* attr, const Pf4Args& p, int rp, int ct, dim3 grid
         case 412: return launch_pf4_t<HP, ZP, 12, 4>(attr, p, grid, st);
         case 409: return launch_pf4_t<HP, ZP, 9, 4>(attr, p, grid, st);
         case 408: return launch_pf4_t<HP, ZP, 8, 4>(attr, p, grid, st);
-        case 405: return launch_pf4_t<HP, ZP, 5, 4>(attr, p, grid, st);
         case 404: return launch_pf4_t<HP, ZP, 4, 4>(attr, p, grid, st);
         case 216: return launch_pf4_t<HP, ZP, 16, 2>(attr, p, grid, st);
         case 208: return launch_pf4_t<HP, ZP, 8, 2>(attr, p, grid, st);

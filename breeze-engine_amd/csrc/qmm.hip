@@ -1193,6 +1193,20 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //     and the block-integer export).
 //   pick_pf_rp  32-row prefill workgroups up to 32 rows, 64 up to 64, then
 //     128 (the C4 shape's 512 rows fill the CUs with 128-row workgroups).
+//   kPf16TilesPerCu (13), kPf16DeepPerCu (6)  the INT4 prefill runs as
+//     independent 16-row waves (pf16_kernel) up to 13 output tiles of 16x16 a
+//     CU, with four weight chunks in flight up to 6 tiles a CU and two past
+//     that (more waves then fit a SIMD).  Workgroups of 32-row waves
+//     (pf4_kernel, best shape) against independent waves, K=5120: N=5120 at 33
+//     / 64 / 128 / 256 rows (4 / 5 / 10 / 20 tiles a CU) 46 / 46 / 48 / 63 ->
+//     29 / 33 / 45 / 78; N=17408 at 33 / 64 rows (13 / 17) 62 / 61 -> 58 / 79;
+//     four chunks against two: N=5120 at 64 / 128 rows 33 / 49 against 39 / 45.
+//   kPf4Start (0.6)  the workgroup shape of the rest (pick_pf4): a call takes
+//     about 40 us + 25 us a column group of the busiest wave at K=5120 (N=17408
+//     at 64 / 128 / 256 / 512 rows, shapes (2, 8) / (4, 8) / (4, 9) / (4, 17):
+//     61 / 82 / 104 / 162), and as much again for a second round; five tiles a
+//     workgroup leave half a group empty (N=17408 at 128 rows 84.7 against
+//     82.3 on eight, N=5120 at 512 rows 100 against 92).
 //   kStreamIdleDiv (8)  plain decode calls read their weight chunks with
 //     non-temporal loads when at most one in 8 of a tile's producer slots
 //     (15 a phase) is idle.  Weights are read once a call; the hint streams
@@ -1239,7 +1253,8 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 // row limit), BREEZE_HIP_DEC8 (0: never the eight-row groups; 2: they take
 // every prologue-quantized call), BREEZE_HIP_DEC8_ROWS (their row limit),
 // BREEZE_HIP_DEC8_LREC (0: records never in LDS; n: from n tiles),
-// BREEZE_HIP_PREFILL_RP / _CT (prefill workgroup shape), BREEZE_HIP_FUSED_MAX_BLOCKS
+// BREEZE_HIP_PREFILL_RP / _CT (prefill workgroup shape), BREEZE_HIP_PF16 (the
+// INT4 prefill's independent waves: 0 never, 1 always), BREEZE_HIP_FUSED_MAX_BLOCKS
 // (row-blocks the decode prologue quantizes), BREEZE_HIP_SPLIT (split-K),
 // BREEZE_HIP_STREAM (non-temporal weight loads), BREEZE_HIP_FLOW (phases
 // across tile boundaries).
@@ -1462,11 +1477,12 @@ void pick_pf4(Plan& p, int M, int tiles, int n_cu) {
     bool rp_ok = false, ct_ok = false;
     for (const PfCfg& c : kPfCfgs) {
         rp_ok = rp_ok || c.rp == rp;
-        ct_ok = ct_ok || ((!rp || c.rp == rp) && c.ct == ct);
+        ct_ok = ct_ok || ((!rp || c.rp == rp) && c.ct == ct && ct != 5);
     }
     double best = -1.0;
     for (const PfCfg& c : kPfCfgs) {
         if ((rp_ok && c.rp != rp) || (ct_ok && c.ct != ct)) continue;
+        if (c.ct == 5) continue;  // half of its third column group is empty: (4, 8) is faster wherever it fits
         const int groups = (c.ct + 1) / 2, parts = std::min(groups, kPfWaves / c.rp), waves_wg = c.rp * parts;
         const int per_cu = std::max(1, kPfWaves / waves_wg);
         int simd = 0;  // column groups on the busiest SIMD of a CU

@@ -327,6 +327,33 @@ __global__ __launch_bounds__(256) void quantize_rec_kernel(const float* __restri
     if (o == 0) *reinterpret_cast<float*>(rec + kRecA + (b * 16 + r) * 4) = s;
 }
 
+// Activation records of the INT8 GEMM for few output tiles (r16_rec_bytes): a
+// wave per (16 rows, block); padding rows are zeros.
+template <bool HP>
+__global__ __launch_bounds__(256) void quantize_r16_kernel(const float* __restrict__ A, int M, int K, int nblk, int nch,
+                                                           int tiles, uint8_t* __restrict__ R) {
+    const int g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int o = lane & 3, r = lane >> 2;
+    const int mt = g / nblk, j = g - mt * nblk, m = 16 * mt + r;
+    if (mt >= tiles) return;  // whole waves only: the quad reductions need all lanes
+    float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f), v1 = v0;
+    if (m < M) {
+        const float* src = A + (size_t)m * K + 32 * j + 8 * o;
+        v0 = *reinterpret_cast<const float4*>(src);
+        v1 = *reinterpret_cast<const float4*>(src + 4);
+    }
+    float s;
+    uint2 ph, pl;
+    quant4x8<HP>(v0, v1, s, ph, pl);
+    // Row 4 o + (r & 3)'s scale, from lane 0 of that row's quad.
+    const float sr = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (4 * (4 * o + (r & 3))), __float_as_int(s)));
+    uint8_t* rec = R + ((size_t)mt * nch + (j >> 1)) * r16_rec_bytes(HP);
+    const int l = r + 16 * o, b = j & 1;
+    if (HP) *reinterpret_cast<uint4*>(rec + 1024 * b + 16 * l) = make_uint4(ph.x, ph.y, pl.x, pl.y);
+    else *reinterpret_cast<uint2*>(rec + 16 * l + 8 * b) = ph;
+    *reinterpret_cast<float*>(rec + (HP ? 2048 : 1024) + 8 * l + 4 * b) = sr;
+}
+
 // Activation records for the INT4 prefill GEMM (kF6Rec): a wave per
 // (16 rows, block); the 4 lanes of a row quantize one block, exchange the
 // base-16 digits of their octets, and lane d packs digit d of the row's 32
@@ -1193,6 +1220,11 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //     and the block-integer export).
 //   pick_pf_rp  32-row prefill workgroups up to 32 rows, 64 up to 64, then
 //     128 (the C4 shape's 512 rows fill the CUs with 128-row workgroups).
+//   kPf16TilesPerCu8 (13)  the same for INT8 (pf16_w8_kernel).  Workgroups
+//     (prefill_kernel) against independent waves, K=5120: N=5120 at 33 / 64 /
+//     128 / 200 rows (4 / 5 / 10 / 16 tiles a CU) 47 / 47 / 58 / 60 -> 21 / 32 /
+//     44 / 70; N=17408 at 32 / 48 / 64 rows (9 / 13 / 17) 46 / 63 / 63 -> 45 /
+//     57 / 67; K=17408 N=5120 at 48 rows 145 -> 59.
 //   kPf16TilesPerCu (13), kPf16DeepPerCu (6)  the INT4 prefill runs as
 //     independent 16-row waves (pf16_kernel) up to 13 output tiles of 16x16 a
 //     CU, with four weight chunks in flight up to 6 tiles a CU and two past
@@ -1254,7 +1286,7 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 // every prologue-quantized call), BREEZE_HIP_DEC8_ROWS (their row limit),
 // BREEZE_HIP_DEC8_LREC (0: records never in LDS; n: from n tiles),
 // BREEZE_HIP_PREFILL_RP / _CT (prefill workgroup shape), BREEZE_HIP_PF16 (the
-// INT4 prefill's independent waves: 0 never, 1 always), BREEZE_HIP_FUSED_MAX_BLOCKS
+// prefill's independent waves: 0 never, 1 always), BREEZE_HIP_FUSED_MAX_BLOCKS
 // (row-blocks the decode prologue quantizes), BREEZE_HIP_SPLIT (split-K),
 // BREEZE_HIP_STREAM (non-temporal weight loads), BREEZE_HIP_FLOW (phases
 // across tile boundaries).
@@ -1266,7 +1298,7 @@ constexpr int kPairMaxRows4 = 16;
 constexpr int kDec8LrecTiles = 2;
 constexpr int kPrefillMinRows = 9;
 constexpr int kSplitMaxTiles = 8, kSplitMinPhases = 20;
-constexpr int kPf16TilesPerCu = 13, kPf16DeepPerCu = 6;
+constexpr int kPf16TilesPerCu = 13, kPf16TilesPerCu8 = 13, kPf16DeepPerCu = 6;
 constexpr double kPf4Start = 0.6;
 constexpr int kStreamIdleDiv = 8, kStreamMaxGroups = 2;
 
@@ -1454,25 +1486,29 @@ int split_pieces(const Shape& h, int M, const CallKind& k, int n_cu, int* lds) {
     return S;
 }
 
-// The INT4 prefill launch (see the routing table): independent 16-row waves up
-// to kPf16TilesPerCu output tiles a CU, else the workgroup shape whose
-// rounds x (half the column groups of a CU's busiest SIMD + kPf4Start) is
-// least; a CU holds eight waves.  BREEZE_HIP_PREFILL_RP / _CT force a workgroup shape,
-// BREEZE_HIP_PF16=0 / 1 turns the independent waves off / on.
+// Whether a prefill call of few output tiles a CU runs as independent 16-row
+// waves (see the routing table).  BREEZE_HIP_PF16=0 / 1 turns them off / on; a
+// forced workgroup shape turns them off.
+bool pick_pf16(Plan& p, int bits, int M, int tiles, int n_cu) {
+    const char* env = std::getenv("BREEZE_HIP_PF16");
+    const long waves = (long)tiles * ((M + 15) / 16);
+    const long most = (long)(bits == 4 ? kPf16TilesPerCu : kPf16TilesPerCu8) * n_cu;
+    const bool few = waves <= most && !std::getenv("BREEZE_HIP_PREFILL_RP") && !std::getenv("BREEZE_HIP_PREFILL_CT");
+    if (!(env ? env[0] == '1' : few)) return false;
+    p.pf_rp = 0;
+    p.pf_ct = 1;
+    p.pf_ahead = waves <= (long)kPf16DeepPerCu * n_cu ? 4 : 2;
+    p.grid_x = (int)((waves + kPf16Waves - 1) / kPf16Waves);
+    p.grid_y = 1;
+    return true;
+}
+
+// The INT4 prefill's workgroup shape: the one whose rounds x (half the column
+// groups of a CU's busiest SIMD + kPf4Start) is least; a CU holds eight waves.
+// BREEZE_HIP_PREFILL_RP / _CT force a shape.
 void pick_pf4(Plan& p, int M, int tiles, int n_cu) {
     const char* frp = std::getenv("BREEZE_HIP_PREFILL_RP");
     const char* fct = std::getenv("BREEZE_HIP_PREFILL_CT");
-    const char* f16 = std::getenv("BREEZE_HIP_PF16");
-    const long waves = (long)tiles * ((M + 15) / 16);
-    const bool few = waves <= (long)kPf16TilesPerCu * n_cu && !frp && !fct;
-    if (f16 ? f16[0] == '1' : few) {
-        p.pf_rp = 0;
-        p.pf_ct = 1;
-        p.pf_ahead = waves <= (long)kPf16DeepPerCu * n_cu ? 4 : 2;
-        p.grid_x = (int)((waves + 3) / 4);
-        p.grid_y = 1;
-        return;
-    }
     const int rp = frp ? std::atoi(frp) : 0, ct = fct ? std::atoi(fct) : 0;
     bool rp_ok = false, ct_ok = false;
     for (const PfCfg& c : kPfCfgs) {
@@ -1564,6 +1600,7 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
         const int rows = 32 * p.pf_rp;
         p.Mpad = (M + rows - 1) / rows * rows;
         p.grid_y = p.Mpad / rows;
+        if (pick_pf16(p, h.bits, M, tiles, n_cu)) return p;
         if (h.bits == 4) {
             pick_pf4(p, M, tiles, n_cu);
             return p;
@@ -1705,6 +1742,14 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
             const unsigned qb = (unsigned)((waves + 3) / 4);
             if (hp) quantize_f6_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, rtiles, mult, s.rec);
             else quantize_f6_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, rtiles, mult, s.rec);
+        } else if (p.pf_rp == 0) {
+            const int rtiles = (M + 15) / 16;
+            const size_t bytes = s.fixed ? int8_bytes : (size_t)rtiles * nch_rec * r16_rec_bytes(hp);
+            if (!grow(w, st, &s.rec, &s.rec_cap, bytes, "workspace alloc", s.fixed)) return -4;
+            const size_t waves = (size_t)rtiles * h->nblk;
+            const unsigned qb = (unsigned)((waves + 3) / 4);
+            if (hp) quantize_r16_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, rtiles, s.rec);
+            else quantize_r16_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, rtiles, s.rec);
         } else {
             if (!grow(w, st, &s.rec, &s.rec_cap, int8_bytes, "workspace alloc", s.fixed)) return -4;
             const size_t threads = (size_t)(p.Mpad / 16) * nch_rec * 2 * 64;  // a wave per (16 rows, block)
@@ -1914,8 +1959,9 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
             pa.sc_shift = h->sc_shift;
             pa.ntiles = h->N / 16;
             const int scm = h->sc_blk ? 2 : (h->sc_shift == 31 ? 0 : 1);
-            e = hp ? launch_pf<true>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st)
-                   : launch_pf<false>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st);
+            if (p.pf_rp == 0) e = launch_pf16_w8(pa, hp, scm, p.grid_x, st);
+            else e = hp ? launch_pf<true>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st)
+                        : launch_pf<false>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st);
         }
     } else {
         const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y);

@@ -804,6 +804,16 @@ __device__ inline uint32_t uniform_offset(uint32_t x) {
     return x;
 }
 
+// Independent waves a workgroup of the kernels for few output tiles (pf16_kernel,
+// pf16_w8_kernel).
+constexpr int kPf16Waves = 4;
+// Activation record of pf16_w8_kernel per (16 rows, chunk of two blocks), in
+// the operand order of v_mfma_i32_16x16x32_i8 (lane r + 16 o: k-octet o of row
+// r).  Two-pass: per block 64 lanes x [8 h bytes, 8 l bytes]; INT8
+// activations: 64 lanes x [8 bytes of block 0, 8 of block 1].  Then 64 lanes x
+// the two block scales of row 4 o + (r & 3), the row of result r & 3.
+__host__ __device__ constexpr int r16_rec_bytes(bool hp) { return hp ? 2560 : 1536; }
+
 struct Pf4Args {
     const char* W;  // [ntiles][nbg][64 lanes][16 B]
     const char* S;  // scales: of (tile t, column c, block j) at t s_tile + (4 (j / 4) >> sc_shift) s_grp + c s_col + (j & 3) s_blk
@@ -882,6 +892,7 @@ hipError_t launch_dec8(bool* attr_set, const GemvArgs& a, const uint4* rec, int 
 template <bool HP>
 hipError_t launch_pf(bool* pf_attr, const PfArgs& p, int scm, int rp, int ct, dim3 grid, hipStream_t st);
 hipError_t launch_pf16(const Pf4Args& p, bool zp, int ahead, int grid, hipStream_t st);
+hipError_t launch_pf16_w8(const PfArgs& p, bool hp, int scm, int grid, hipStream_t st);
 template <bool HP>
 hipError_t launch_pf4(bool* pf_attr, const Pf4Args& p, bool zp, int rp, int ct, dim3 grid, hipStream_t st);
 

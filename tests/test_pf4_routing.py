@@ -1,6 +1,6 @@
-"""Which launch an INT4 prefill call takes (pick_pf4 in csrc/qmm.hip): few
-output tiles a CU go to independent 16-row waves (pf_rp 0), more to the
-workgroup shape with the fewest rounds of column groups."""
+"""Which launch a prefill call takes (pick_pf16, pick_pf4 in csrc/qmm.hip): few
+output tiles a CU go to independent 16-row waves (pf_rp 0), more to a
+workgroup shape, for INT4 the one with the fewest rounds of column groups."""
 import pytest
 
 TABLE = [
@@ -33,6 +33,18 @@ def test_overrides(hb, monkeypatch):
     monkeypatch.setenv("BREEZE_HIP_PREFILL_CT", "16")
     p = hb.plan(4, 33, 5120, 5120)
     assert (p["pf_rp"], p["pf_ct"]) == (2, 16)
+
+
+@pytest.mark.parametrize("shape,want", [
+    ((8, 64, 5120, 5120), dict(pf_rp=0, grid_x=320)),
+    ((8, 48, 5120, 17408), dict(pf_rp=0, grid_x=816)),  # 12.75 tiles a CU
+    ((8, 64, 5120, 17408), dict(pf_rp=2)),              # 17
+    ((8, 512, 5120, 17408), dict(pf_rp=4, pf_ct=17)),
+])
+def test_int8_prefill_launch(hb, shape, want):
+    got = hb.plan(*shape, n_cu=256)
+    assert got["route"] == "prefill"
+    assert {k: got[k] for k in want} == want, got
 
 
 @pytest.mark.parametrize("M", [33, 64, 100, 128, 256, 512, 1000, 4096])

@@ -249,12 +249,41 @@ def _prepack_numpy(qweight, scales, qzeros, K, N, bits=4, block_size=32):
 
 
 def _is_torch(x):
-    return type(x).__module__.split(".")[0] == "torch"
+    return type(x) is _tensor or type(x).__module__.split(".")[0] == "torch"
+
+
+# The host's part of a call, kept short: a single-token projection takes the GPU
+# about 5 us, and torch's general forms of these steps (a stream object, a
+# conversion that changes nothing) took the host 9.3 us a call; now 6.
+_torch = None
+_tensor = None  # torch.Tensor
+_raw_stream = None  # device index -> current stream's hipStream_t, where this torch offers it
+
+
+def _import_torch():
+    global _torch, _tensor, _raw_stream
+    if _torch is None:
+        import torch
+
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        _tensor = torch.Tensor
+        _torch = torch
+    return _torch
+
+
+def _f32(t):
+    """`t` as a contiguous fp32 tensor (itself when it is one)."""
+    if t.dtype is _torch.float32 and t.is_contiguous():
+        return t
+    return t.to(_torch.float32).contiguous()
 
 
 def _torch_stream(t):
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    torch = _import_torch()
+    dev = t.get_device()  # -1 on the CPU: the general form raises for it
+    if _raw_stream is not None and dev >= 0:
+        return _raw_stream(dev)
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _check_rc(rc, what):
@@ -269,11 +298,11 @@ def matmul(handle, a2d, N):
     a GPU torch tensor out (asynchronous on the current stream)."""
     _require_lib()
     if _is_torch(a2d):
-        import torch
-        a = a2d.to(torch.float32).contiguous()
+        torch = _import_torch()
+        a = _f32(a2d)
         M = a.shape[0]
         out = torch.empty((M, N), dtype=torch.float32, device=a.device)
-        _check_rc(_lib.i4_matmul_dev(_vp(handle), _vp(a.data_ptr()), int(M), _vp(out.data_ptr()),
+        _check_rc(_lib.i4_matmul_dev(_vp(handle), a.data_ptr(), int(M), out.data_ptr(),
                                      _torch_stream(a)), "i4_matmul_dev")
         return out
     a2d = np.ascontiguousarray(a2d, dtype=np.float32)
@@ -291,11 +320,11 @@ def matmul_silu_mul(gate, up, a2d, N):
     decoder MLP's gate/up step (kernel/qwen35_decoder.cpp:406-408) in one
     call, asynchronous on the current stream."""
     _require_lib()
-    import torch
-    a = a2d.to(torch.float32).contiguous()
+    torch = _import_torch()
+    a = _f32(a2d)
     M = a.shape[0]
     out = torch.empty((M, N), dtype=torch.float32, device=a.device)
-    _check_rc(_lib.i4_matmul_silu_mul_dev(_vp(gate), _vp(up), _vp(a.data_ptr()), int(M), _vp(out.data_ptr()),
+    _check_rc(_lib.i4_matmul_silu_mul_dev(_vp(gate), _vp(up), a.data_ptr(), int(M), out.data_ptr(),
                                           _torch_stream(a)), "i4_matmul_silu_mul_dev")
     return out
 
@@ -327,13 +356,13 @@ def silu_mul(g, u):
     MLP's elementwise step (kernel/qwen35_decoder.cpp:408) bit for bit,
     asynchronous on the current stream."""
     _require_lib()
-    import torch
-    g = g.to(torch.float32).contiguous()
-    u = u.to(torch.float32).contiguous()
+    torch = _import_torch()
+    g = _f32(g)
+    u = _f32(u)
     if g.shape != u.shape:
         raise ValueError(f"silu_mul: shapes {tuple(g.shape)} and {tuple(u.shape)} differ")
     out = torch.empty_like(g)
-    _check_rc(_lib.i4_silu_mul_dev(_vp(g.data_ptr()), _vp(u.data_ptr()), g.numel(), _vp(out.data_ptr()),
+    _check_rc(_lib.i4_silu_mul_dev(g.data_ptr(), u.data_ptr(), g.numel(), out.data_ptr(),
                                    _torch_stream(g)), "i4_silu_mul_dev")
     return out
 
@@ -344,15 +373,15 @@ def matmul_multi(handles, a2d, Ns):
     in_a (kernel/qwen35_decoder.cpp:285-288), in one launch when they share
     a device layout; asynchronous on the current stream."""
     _require_lib()
-    import torch
+    torch = _import_torch()
     if not 1 <= len(handles) <= 4 or len(handles) != len(Ns):
         raise ValueError("matmul_multi takes 1 to 4 handles and one N per handle")
-    a = a2d.to(torch.float32).contiguous()
+    a = _f32(a2d)
     M = a.shape[0]
     outs = [torch.empty((M, int(n)), dtype=torch.float32, device=a.device) for n in Ns]
     hv = (ctypes.c_void_p * len(handles))(*[int(h) for h in handles])
     cv = (ctypes.c_void_p * len(outs))(*[o.data_ptr() for o in outs])
-    _check_rc(_lib.i4_matmul_multi_dev(hv, len(handles), _vp(a.data_ptr()), int(M), cv, _torch_stream(a)),
+    _check_rc(_lib.i4_matmul_multi_dev(hv, len(handles), a.data_ptr(), int(M), cv, _torch_stream(a)),
               "i4_matmul_multi_dev")
     return outs
 
@@ -364,20 +393,20 @@ def rmsnorm_matmul_multi(x2d, w, eps, handles, Ns, want_hn=False):
     one launch when the decode kernel quantizes the activation itself;
     asynchronous on the current stream."""
     _require_lib()
-    import torch
+    torch = _import_torch()
     if not 1 <= len(handles) <= 4 or len(handles) != len(Ns):
         raise ValueError("rmsnorm_matmul_multi takes 1 to 4 handles and one N per handle")
-    x = x2d.to(torch.float32).contiguous()
+    x = _f32(x2d)
     M, K = x.shape
-    wv = w.to(device=x.device, dtype=torch.float32).contiguous()
+    wv = _f32(w if w.device == x.device else w.to(x.device))
     if wv.numel() != K:
         raise ValueError(f"w has {wv.numel()} elements, x rows have {K}")
     outs = [torch.empty((M, int(n)), dtype=torch.float32, device=x.device) for n in Ns]
     hn = torch.empty_like(x) if want_hn else None
     hv = (ctypes.c_void_p * len(handles))(*[int(h) for h in handles])
     cv = (ctypes.c_void_p * len(outs))(*[o.data_ptr() for o in outs])
-    _check_rc(_lib.i4_rmsnorm_matmul_multi_dev(_vp(x.data_ptr()), _vp(wv.data_ptr()), float(eps), hv, len(handles),
-                                               int(M), cv, _vp(hn.data_ptr()) if want_hn else None,
+    _check_rc(_lib.i4_rmsnorm_matmul_multi_dev(x.data_ptr(), wv.data_ptr(), float(eps), hv, len(handles),
+                                               int(M), cv, hn.data_ptr() if want_hn else None,
                                                _torch_stream(x)), "i4_rmsnorm_matmul_multi_dev")
     return (outs, hn) if want_hn else outs
 
@@ -388,43 +417,43 @@ def rmsnorm(x2d, w, eps):
     current stream.  Its output is the activation of the projections that
     follow (input_ln / post_ln ahead of qkv, gate/up)."""
     _require_lib()
-    import torch
-    x = x2d.to(torch.float32).contiguous()
+    torch = _import_torch()
+    x = _f32(x2d)
     if x.dim() != 2:
         raise ValueError(f"x must be 2-D [s, H], got shape {tuple(x.shape)}")
     s, H = x.shape
-    wv = w.to(device=x.device, dtype=torch.float32).contiguous()
+    wv = _f32(w if w.device == x.device else w.to(x.device))
     if wv.numel() != H:
         raise ValueError(f"w has {wv.numel()} elements, x rows have {H}")
     out = torch.empty_like(x)
     if s == 0:
         return out
-    _check_rc(_lib.i4_rmsnorm_dev(_vp(x.data_ptr()), _vp(wv.data_ptr()), int(s), int(H), float(eps),
-                                  _vp(out.data_ptr()), _torch_stream(x)), "i4_rmsnorm_dev")
+    _check_rc(_lib.i4_rmsnorm_dev(x.data_ptr(), wv.data_ptr(), int(s), int(H), float(eps),
+                                  out.data_ptr(), _torch_stream(x)), "i4_rmsnorm_dev")
     return out
 
 
 def matmul_argmax(handle, a2d, N):
     """GPU torch tensor [M, K] -> (logits fp32 [M, N], argmax int64 [M])."""
     _require_lib()
-    import torch
-    a = a2d.to(torch.float32).contiguous()
+    torch = _import_torch()
+    a = _f32(a2d)
     M = a.shape[0]
     out = torch.empty((M, N), dtype=torch.float32, device=a.device)
     idx = torch.empty((M,), dtype=torch.int64, device=a.device)
-    _check_rc(_lib.i4_matmul_argmax_dev(_vp(handle), _vp(a.data_ptr()), int(M), _vp(out.data_ptr()),
-                                        _vp(idx.data_ptr()), _torch_stream(a)), "i4_matmul_argmax_dev")
+    _check_rc(_lib.i4_matmul_argmax_dev(_vp(handle), a.data_ptr(), int(M), out.data_ptr(),
+                                        idx.data_ptr(), _torch_stream(a)), "i4_matmul_argmax_dev")
     return out, idx
 
 
 def block_dots(handle, a2d, N, K):
     """GPU torch tensor [M, K] -> int32 [M, N, K/32] exact block integers."""
     _require_lib()
-    import torch
-    a = a2d.to(torch.float32).contiguous()
+    torch = _import_torch()
+    a = _f32(a2d)
     M = a.shape[0]
     cs = torch.empty((M, N, K // 32), dtype=torch.int32, device=a.device)
-    _check_rc(_lib.i4_block_dots_dev(_vp(handle), _vp(a.data_ptr()), int(M), _vp(cs.data_ptr()),
+    _check_rc(_lib.i4_block_dots_dev(_vp(handle), a.data_ptr(), int(M), cs.data_ptr(),
                                      _torch_stream(a)), "i4_block_dots_dev")
     return cs
 

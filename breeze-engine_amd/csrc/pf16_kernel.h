@@ -33,19 +33,22 @@ __global__ __launch_bounds__(kPf16Waves * 64, AHEAD == 2 ? 4 : 3) void pf16_kern
     char* lds = pf16_lds + wave * 2 * kPf16Stage;
     const int c16 = lane & 15, q4 = lane >> 4;
     const int nst = a.nbg;
+    const int sk = a.find(tile), st = tile - a.first(sk);  // segment, and the tile within it
+    const Pf4Seg& sg = a.seg[sk];
 
     // Weights: after the transpose, lane (column c16, block q4) of the chunk.
     uint4 raw[AHEAD];
     float rsc[AHEAD];
     int rzp[AHEAD];
-    const char* wp = a.W + (size_t)tile * a.nbg * 1024 + 16 * lane;
-    const char* sp = a.S + (size_t)tile * a.s_tile + a.s_col * c16 + a.s_blk * q4;
-    const char* zpp = ZP ? a.Z + (size_t)tile * a.nbg * 64 + 4 * c16 + q4 : nullptr;
+    const gptr wp = uniform_ptr(sg.W + (size_t)st * a.nbg * 1024);
+    const gptr sp = uniform_ptr(sg.S + (size_t)st * a.s_tile);
+    const uint32_t soff = a.s_col * c16 + a.s_blk * q4;
+    const gptr zpp = ZP ? uniform_ptr(sg.Z + (size_t)st * a.nbg * 64) : nullptr;
     auto load_raw = [&](int r, int g) __attribute__((always_inline)) {
         const int gc = min(g, nst - 1);
-        raw[r] = *reinterpret_cast<const uint4*>(wp + (size_t)uniform_offset((uint32_t)gc) * 1024);
-        rsc[r] = *reinterpret_cast<const float*>(sp + (size_t)uniform_offset((uint32_t)((4 * gc) >> a.sc_shift)) * a.s_grp);
-        if (ZP) rzp[r] = (int8_t)zpp[(size_t)uniform_offset((uint32_t)gc) * 64];
+        raw[r] = __builtin_bit_cast(uint4, gload<v4u>(wp + (size_t)uniform_offset((uint32_t)gc) * 1024 + (uint32_t)(16 * lane)));
+        rsc[r] = gload<float>(sp + (size_t)uniform_offset((uint32_t)((4 * gc) >> a.sc_shift)) * a.s_grp + soff);
+        if (ZP) rzp[r] = gload<int8_t>(zpp + (size_t)uniform_offset((uint32_t)gc) * 64 + (uint32_t)(4 * c16 + q4));
     };
     auto expand = [&](int r, char* eb) __attribute__((always_inline)) {
         uint32_t w[4], d[6];
@@ -142,11 +145,11 @@ __global__ __launch_bounds__(kPf16Waves * 64, AHEAD == 2 ? 4 : 3) void pf16_kern
         block(bp0 + (nfull & 1) * kPf16Stage, b & 3, ab[0]);
     }
     epi();
-    const int n = tile * 16 + c16;
+    const int n = st * 16 + c16;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int m = 16 * rt + 4 * q4 + j;
-        if (m < a.M) a.C[(size_t)m * a.N + n] = acc[j];
+        if (m < a.M) sg.C[(size_t)m * sg.N + n] = acc[j];
     }
 }
 

@@ -56,13 +56,21 @@ __global__ __launch_bounds__((Pf4Shape<CT, RP>::kThreads)) void pf4_kernel(Pf4Ar
     float rsc[SLOTS];
     int rzp[SLOTS];
     const uint32_t soff = a.s_col * ec + a.s_blk * ej;
+    // The tile slots' weights (scales, zero points).
+    gptr wt[SLOTS], stp[SLOTS], zt[SLOTS];
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        const int t = min(t0 + wave + L::kWaves * i, a.ntiles - 1), k = a.find(t);
+        const size_t ts = t - a.first(k);
+        wt[i] = uniform_ptr(a.seg[k].W + ts * a.nbg * 1024);
+        stp[i] = uniform_ptr(a.seg[k].S + ts * a.s_tile);
+        zt[i] = ZP ? uniform_ptr(a.seg[k].Z + ts * a.nbg * 64) : nullptr;
+    }
     auto load_raw = [&](int i, int g) __attribute__((always_inline)) {
-        const int u = wave + L::kWaves * i;
-        const int tc = min(t0 + u, a.ntiles - 1), gc = min(g, nst - 1);
-        raw[i] = *reinterpret_cast<const uint4*>(a.W + ((size_t)tc * a.nbg + gc) * 1024 + 16 * lane);
-        const char* s = a.S + (size_t)tc * a.s_tile + (size_t)((4 * gc) >> a.sc_shift) * a.s_grp;
-        rsc[i] = *reinterpret_cast<const float*>(s + soff);
-        if (ZP) rzp[i] = (int8_t)(a.Z + ((size_t)tc * a.nbg + gc) * 64)[4 * ec + ej];
+        const uint32_t gc = (uint32_t)min(g, nst - 1);
+        raw[i] = __builtin_bit_cast(uint4, gload<v4u>(wt[i] + (size_t)uniform_offset(gc) * 1024 + (uint32_t)(16 * lane)));
+        rsc[i] = gload<float>(stp[i] + (size_t)uniform_offset((4 * gc) >> a.sc_shift) * a.s_grp + soff);
+        if (ZP) rzp[i] = gload<int8_t>(zt[i] + (size_t)uniform_offset(gc) * 64 + (uint32_t)(4 * ec + ej));
     };
     // Expands tile slot i of a stage into the operand buffer eb: two 16-byte
     // planes per (column group, block), so sixteen lanes write and read 256
@@ -258,10 +266,13 @@ __global__ __launch_bounds__((Pf4Shape<CT, RP>::kThreads)) void pf4_kernel(Pf4Ar
         for (int g = 0; g < NG; ++g) {
             const int ct = 2 * (g0 + g) + (c32 >> 4), tile = t0 + ct;
             if (ct >= CT || tile >= a.ntiles) continue;
+            const int k = a.find(tile);
+            float* c = a.seg[k].C + (tile - a.first(k)) * 16 + (c32 & 15);
+            const int n = a.seg[k].N;
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
                 const int m = rpair * 32 + (j & 3) + 8 * (j >> 2) + 4 * kh;
-                if (m < a.M) a.C[(size_t)m * a.N + tile * 16 + (c32 & 15)] = acc[g][j];
+                if (m < a.M) c[(size_t)m * n] = acc[g][j];
             }
         }
     };

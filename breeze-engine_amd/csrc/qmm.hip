@@ -1233,6 +1233,13 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //     / 64 / 128 / 256 rows (4 / 5 / 10 / 20 tiles a CU) 46 / 46 / 48 / 63 ->
 //     29 / 33 / 45 / 78; N=17408 at 33 / 64 rows (13 / 17) 62 / 61 -> 58 / 79;
 //     four chunks against two: N=5120 at 64 / 128 rows 33 / 49 against 39 / 45.
+//   paired and multi-projection calls past 32 rows  one INT4 prefill launch
+//     over all projections' tiles (two launches each, records and GEMM,
+//     before).  K=5120, with the INT8-MFMA GEMM then -> now: gate/up (N=17408)
+//     with SiLU at 33 / 200 / 512 rows 162 / 259 / 457 -> 91 / 162 / 344 (207 at
+//     200 rows as two launches of this kernel); RMSNorm + in_qkv/z/b/a at 33 /
+//     128 / 300 rows 247 / 283 / 345 -> 62 / 88 / 131; q/k/v 183 / 208 / 306 ->
+//     44 / 63 / 112.
 //   kPf4Start (0.6)  the workgroup shape of the rest (pick_pf4): a call takes
 //     about 40 us + 25 us a column group of the busiest wave at K=5120 (N=17408
 //     at 64 / 128 / 256 / 512 rows, shapes (2, 8) / (4, 8) / (4, 9) / (4, 17):
@@ -1558,6 +1565,18 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
         return p;
     }
     const bool fz = k.pair || k.multi;
+    // Past the decode rows the projections of one activation share one INT4
+    // prefill launch: their tiles together fill the CUs better than each alone
+    // (see the routing table), and the records are made once.
+    if (fz && M > kDec8MaxRows && h.bits == 4 && !k.norm && !k.argmax && !k.dots && !h.has_dl) {
+        p.route = kRoutePrefill;
+        p.quant = kQuantPrefill;
+        const int tiles = (k.tiles > 0 ? k.tiles : ntiles) * (k.pair ? 2 : 1);
+        const int rows = 32 * pick_pf_rp(M, nullptr);
+        p.Mpad = (M + rows - 1) / rows * rows;
+        if (!pick_pf16(p, h.bits, M, tiles, n_cu)) pick_pf4(p, M, tiles, n_cu);
+        return p;
+    }
     int Mr_max = std::min(M, 4);
     // One or two rows: block pairs per MFMA when that record layout fits.
     const int lds_p64 = (M <= 2 && !k.dots) ? plan_dec_lds(h.nblk, Mr_max, JG, true) : 0;
@@ -1726,6 +1745,13 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
     }
     const Plan p = plan_call(shape_of(h), M, kind, device_cus(w, dev));
     if (p.route == kRouteNone) return kNotPairable;
+    if (p.route == kRoutePrefill && (h2 || mp)) {
+        // One prefill launch for all (the gate's product and the SiLU follow).
+        bool dl = h2 && h2->has_dl;
+        for (int k = 0; mp && k < mp->n; ++k) dl = dl || mp->h[k]->has_dl;
+        if (dl) return kNotPairable;
+        if (h2 && !grow(w, st, &s.gate, &s.gate_cap, (size_t)M * h->N, "workspace alloc")) return -4;
+    }
 
     // The stand-alone quantizer ahead of the matmul kernel.
     if (p.quant == kQuantPrefill) {
@@ -1917,16 +1943,24 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
         const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y);
         if (h->bits == 4) {
             Pf4Args pa{};
-            pa.W = reinterpret_cast<const char*>(h->W);
-            pa.S = reinterpret_cast<const char*>(h->S);
-            pa.Z = reinterpret_cast<const char*>(h->Z);
             pa.R = reinterpret_cast<const char*>(s.rec);
-            pa.C = dC;
             pa.M = M;
-            pa.N = h->N;
             pa.nblk = h->nblk;
             pa.nbg = h->nbg;
-            pa.ntiles = h->N / 16;
+            for (int k = 0; k < kMaxSeg; ++k) pa.seg[k].end = std::numeric_limits<int>::max();
+            auto segment = [&](int k, const Handle* hk, float* c) {
+                pa.ntiles += hk->N / 16;
+                pa.seg[k] = Pf4Seg{reinterpret_cast<const char*>(hk->W), reinterpret_cast<const char*>(hk->S),
+                                   reinterpret_cast<const char*>(hk->Z), c, hk->N, pa.ntiles};
+            };
+            if (mp) {
+                for (int k = 0; k < mp->n; ++k) segment(k, mp->h[k], mp->C[k]);
+            } else if (pair) {
+                segment(0, h, s.gate);
+                segment(1, h2, dC);
+            } else {
+                segment(0, h, dC);
+            }
             if (h->sc_blk) {  // [tile][chunk][16][4]
                 pa.sc_shift = 2;
                 pa.s_tile = (size_t)h->nbg * 256;
@@ -1971,6 +2005,11 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
     }
     if (!hip_ok(e, "matmul launch")) return -5;
 
+    if (pair && p.route == kRoutePrefill) {
+        const size_t n = (size_t)M * h->N;
+        silu_mul_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(s.gate, dC, dC, n);
+        if (!hip_ok(hipGetLastError(), "silu-mul launch")) return -5;
+    }
     if (dIdx && !dots && !decode) {
         // Both decode kernels merge their own argmax (last workgroup).
         const int nparts = (h->N + kArgmaxChunk - 1) / kArgmaxChunk;

@@ -12,6 +12,7 @@
 #include <type_traits>
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
 namespace bq {
 
@@ -814,16 +815,44 @@ constexpr int kPf16Waves = 4;
 // the two block scales of row 4 o + (r & 3), the row of result r & 3.
 __host__ __device__ constexpr int r16_rec_bytes(bool hp) { return hp ? 2560 : 1536; }
 
-struct Pf4Args {
-    const char* W;  // [ntiles][nbg][64 lanes][16 B]
+// A uniform pointer to global memory, in scalar registers.  Pointers picked
+// from an argument array are generic otherwise, and their loads flat.
+typedef const __attribute__((address_space(1))) char* gptr;
+__device__ inline gptr uniform_ptr(const void* p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (gptr)((uint64_t)hi << 32 | lo);
+}
+template <typename T>
+__device__ inline T gload(gptr p) {
+    typedef T GT __attribute__((address_space(1)));
+    return *(const GT*)p;
+}
+
+// One projection of a launch.
+struct Pf4Seg {
+    const char* W;  // [tiles][nbg][64 lanes][16 B]
     const char* S;  // scales: of (tile t, column c, block j) at t s_tile + (4 (j / 4) >> sc_shift) s_grp + c s_col + (j & 3) s_blk
-    const char* Z;  // per-block zero points [ntiles][nbg][16][4], or NULL (8 everywhere)
-    const char* R;  // activation records [16-row tiles][nblk]
+    const char* Z;  // per-block zero points [tiles][nbg][16][4], or NULL (8 everywhere)
     float* C;       // [M][N]
-    int M, N, nblk, nbg, ntiles, sc_shift;
+    int N;
+    int end;        // tiles of this and the segments before it (unused segments: INT_MAX)
+};
+
+// Projections of one activation in one launch: the segments' column tiles are
+// numbered through (kMaxSeg; one layout, all but N alike).
+struct Pf4Args {
+    const char* R;  // activation records [16-row tiles][nblk]
+    int M, nblk, nbg, ntiles, sc_shift;
     int s_grp, s_col, s_blk;
     size_t s_tile;
+    Pf4Seg seg[kMaxSeg];
+    // The segment of tile t, and the segment's first tile.
+    __device__ int find(int t) const { return (t >= seg[0].end) + (t >= seg[1].end) + (t >= seg[2].end); }
+    __device__ int first(int k) const { return k == 0 ? 0 : k == 1 ? seg[0].end : k == 2 ? seg[1].end : seg[2].end; }
 };
+static_assert(kMaxSeg == 4, "Pf4Args::find");
 
 // A workgroup of RP row pairs (32 rows each) by CT column tiles: groups of two
 // tiles (32 columns) split over kParts waves per row pair.

@@ -97,8 +97,8 @@ int i4_matmul_argmax_dev(void* handle, const float* dA, int M, float* dC,
  * Both projections are bit-identical to i4_matmul_dev's, and the SiLU and
  * product are the reference's bit for bit (its expf, the host C library's,
  * restated on the device).  When a decode launch takes both projections it
- * is one launch (SiLU and product in the epilogue); otherwise two launches
- * and i4_silu_mul_dev's kernel.  Returns as i4_matmul_dev. */
+ * is one launch (SiLU and product in the epilogue); otherwise one INT4
+ * prefill launch past 32 rows, or two launches, and i4_silu_mul_dev's kernel.  Returns as i4_matmul_dev. */
 int i4_matmul_silu_mul_dev(void* gate, void* up, const float* dA, int M, float* dC, void* stream);
 
 /* The decoder MLP's elementwise step on device pointers, replacing the loop
@@ -135,7 +135,8 @@ int i4_matmul_noalloc_dev(void* handle, const float* dA, int M, float* dC, int64
  * of one device layout (all but N alike, no per-block metadata) it is one
  * decode launch whose workgroups share out the concatenated column tiles
  * (the activation is quantized once per workgroup, and small projections
- * ride along with large ones); otherwise one launch per handle.  Returns as
+ * ride along with large ones); INT4 handles past 32 rows likewise share one
+ * prefill launch; otherwise one launch per handle.  Returns as
  * i4_matmul_dev. */
 int i4_matmul_multi_dev(void* const* handles, int n, const float* dA, int M, float* const* dC, void* stream);
 
@@ -163,8 +164,8 @@ int i4_rmsnorm_matmul_multi_dev(const float* dX, const float* dNormW, float eps,
  * stand-alone quantizer (0 none: the decode prologue quantizes, 1 staged
  * records, 2 eight-row records, 3 prefill records), prologue quantizes,
  * block pairs, records in LDS, rows per row group, row groups, tile ranges,
- * row groups of a tile range on one XCD, LDS bytes, prefill row pairs,
- * prefill column tiles, grid x, grid y, split-K workgroups per tile (0:
+ * row groups of a tile range on one XCD, LDS bytes, prefill row pairs
+ * (0: independent 16-row waves), prefill column tiles, grid x, grid y, split-K workgroups per tile (0:
  * none), non-temporal weight loads, phases across tile boundaries.
  * Environment overrides apply as for
  * a call.  Returns the number of values written (at most nout), or -1. */

@@ -47,6 +47,21 @@ def test_int8_prefill_launch(hb, shape, want):
     assert {k: got[k] for k in want} == want, got
 
 
+def test_projections_share_a_prefill_launch(hb):
+    """Past 32 rows the gate/up pair (twice the tiles) and multi-projection
+    calls take one INT4 prefill launch; INT8 ones, the fused norm, argmax and
+    a legacy corr do not."""
+    p = hb.plan(4, 200, 5120, 17408, pair=True)
+    assert (p["route"], p["pf_rp"], p["pf_ct"], p["grid_x"], p["grid_y"]) == ("prefill", 4, 17, 128, 2)
+    assert hb.plan(4, 64, 5120, 10240, multi=True)["route"] == "prefill"
+    assert hb.plan(4, 64, 5120, 10240, multi=True, extra=True)["route"] == "prefill"
+    assert hb.plan(4, 32, 4096, 4096, pair=True)["route"] is None
+    assert hb.plan(8, 64, 5120, 10240, multi=True)["route"] is None
+    assert hb.plan(4, 64, 5120, 10240, multi=True, norm=True)["route"] is None
+    assert hb.plan(4, 64, 5120, 10240, multi=True, argmax=True)["route"] is None
+    assert hb.plan(4, 64, 5120, 10240, pair=True, legacy_corr=True)["route"] is None
+
+
 @pytest.mark.parametrize("M", [33, 64, 100, 128, 256, 512, 1000, 4096])
 @pytest.mark.parametrize("N", [16, 48, 1024, 5120, 17408, 151936])
 def test_every_output_is_covered(hb, M, N):

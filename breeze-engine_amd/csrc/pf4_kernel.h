@@ -262,17 +262,37 @@ __global__ __launch_bounds__((Pf4Shape<CT, RP>::kThreads)) void pf4_kernel(Pf4Ar
         }
         epi(NG - 1, sap, std::integral_constant<int, 0>{});
         epi(NG - 1, sap, std::integral_constant<int, 1>{});
+        // Stores.  The two tiles of a group have uniform numbers, and what is
+        // read of their segments stays in scalar registers: loads and stores
+        // share a counter, so a vector load ahead of a store makes it wait for
+        // every store before it.
+        const int m0 = rpair * 32 + 4 * kh;
+        const bool odd = c32 & 16, whole = rpair * 32 + 32 <= a.M;
+        auto column0 = [&](int t, int& n) __attribute__((always_inline)) {
+            const int k = a.find(t);
+            n = __builtin_amdgcn_readfirstlane(a.seg[k].N);
+            return (gfptr)uniform_ptr(a.seg[k].C + (t - a.first(k)) * 16);
+        };
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
-            const int ct = 2 * (g0 + g) + (c32 >> 4), tile = t0 + ct;
-            if (ct >= CT || tile >= a.ntiles) continue;
-            const int k = a.find(tile);
-            float* c = a.seg[k].C + (tile - a.first(k)) * 16 + (c32 & 15);
-            const int n = a.seg[k].N;
+            const int ct = 2 * (g0 + g), t = t0 + ct;
+            int na, nb;
+            const gfptr ca = column0(min(t, a.ntiles - 1), na), cb = column0(min(t + 1, a.ntiles - 1), nb);
+            const ptrdiff_t n = odd ? nb : na;
+            gfptr c = (odd ? cb : ca) + (c32 & 15) + m0 * n;
+            if (ct + odd >= CT || t + odd >= a.ntiles) continue;
+            if (whole) {
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int m = rpair * 32 + (j & 3) + 8 * (j >> 2) + 4 * kh;
-                if (m < a.M) c[(size_t)m * n] = acc[g][j];
+                for (int j = 0; j < 16; ++j) {
+                    *c = acc[g][j];
+                    c += (j & 3) == 3 ? 5 * n : n;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    if (m0 + (j & 3) + 8 * (j >> 2) < a.M) *c = acc[g][j];
+                    c += (j & 3) == 3 ? 5 * n : n;
+                }
             }
         }
     };

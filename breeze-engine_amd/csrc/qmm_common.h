@@ -818,6 +818,7 @@ __host__ __device__ constexpr int r16_rec_bytes(bool hp) { return hp ? 2560 : 15
 // A uniform pointer to global memory, in scalar registers.  Pointers picked
 // from an argument array are generic otherwise, and their loads flat.
 typedef const __attribute__((address_space(1))) char* gptr;
+typedef __attribute__((address_space(1))) float* gfptr;
 __device__ inline gptr uniform_ptr(const void* p) {
     const uint64_t v = (uint64_t)p;
     const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);

@@ -1339,10 +1339,10 @@ bool dec8_prologue_call(int M, int nblk, int ntiles) {
 // What routing reads of a handle.
 struct Shape {
     int bits, N, nblk, nblk4, nblk_pad;
-    bool extra, has_dl, has_ws;
+    bool extra, has_dl, has_ws, has_zp;
 };
 Shape shape_of(const Handle* h) {
-    return Shape{h->bits, h->N, h->nblk, h->nblk4, h->nblk_pad, h->extra, h->has_dl, h->WS != nullptr};
+    return Shape{h->bits, h->N, h->nblk, h->nblk4, h->nblk_pad, h->extra, h->has_dl, h->WS != nullptr, h->has_zp};
 }
 
 // LDS bytes of the decode kernel for Mr_max rows per row group, or 0 if the
@@ -1422,6 +1422,7 @@ struct Plan {
     // Prefill: row pairs (0: independent 16-row waves), column tiles, padded
     // rows, weight chunks in flight of the independent waves.
     int pf_rp = 0, pf_ct = 0, Mpad = 0, pf_ahead = 0;
+    bool pf_zp = false;      // INT4 prefill: the kernel reads zero points
     int grid_x = 0, grid_y = 1;
     int split = 0;           // decode split-K: workgroups per tile (0: none)
     bool stream = false;     // decode: weight chunks read with non-temporal loads
@@ -1571,6 +1572,7 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
     if (fz && M > kDec8MaxRows && h.bits == 4 && !k.norm && !k.argmax && !k.dots && !h.has_dl) {
         p.route = kRoutePrefill;
         p.quant = kQuantPrefill;
+        p.pf_zp = h.has_zp;
         const int tiles = (k.tiles > 0 ? k.tiles : ntiles) * (k.pair ? 2 : 1);
         const int rows = 32 * pick_pf_rp(M, nullptr);
         p.Mpad = (M + rows - 1) / rows * rows;
@@ -1615,6 +1617,7 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
     if (pre) {
         p.route = kRoutePrefill;
         p.quant = kQuantPrefill;
+        p.pf_zp = h.has_zp;
         p.pf_rp = pick_pf_rp(M, std::getenv("BREEZE_HIP_PREFILL_RP"));
         const int rows = 32 * p.pf_rp;
         p.Mpad = (M + rows - 1) / rows * rows;
@@ -1743,7 +1746,13 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
         kind.tiles = 0;
         for (int k = 0; k < mp->n; ++k) kind.tiles += mp->h[k]->N / 16;
     }
-    const Plan p = plan_call(shape_of(h), M, kind, device_cus(w, dev));
+    // Explicit zero points on any projection of the call.  Per-block scales
+    // alone also give a handle zero points (all 8, Handle::Z), which the INT4
+    // prefill leaves unread: as 8 everywhere they are part of the row sums.
+    Shape shape = shape_of(h);
+    if (h2) shape.has_zp = shape.has_zp || h2->has_zp;
+    for (int k = 0; mp && k < mp->n; ++k) shape.has_zp = shape.has_zp || mp->h[k]->has_zp;
+    const Plan p = plan_call(shape, M, kind, device_cus(w, dev));
     if (p.route == kRouteNone) return kNotPairable;
     if (p.route == kRoutePrefill && (h2 || mp)) {
         // One prefill launch for all (the gate's product and the SiLU follow).
@@ -1759,7 +1768,7 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
         const int nch_rec = (h->nblk + 1) / 2;  // record chunks of two blocks
         const size_t int8_bytes = (size_t)(p.Mpad / 16) * nch_rec * kRecBytes;
         if (h->bits == 4) {
-            const int rtiles = (M + 31) / 32 * 2, mult = h->Z ? 1 : 8;
+            const int rtiles = (M + 31) / 32 * 2, mult = p.pf_zp ? 1 : 8;
             // The fixed scratch counts the INT8 records' bytes (the array is
             // larger by the FP6 records' share, kNoAllocArray).
             const size_t bytes = s.fixed ? int8_bytes : (size_t)rtiles * h->nblk * kF6Rec;
@@ -1974,10 +1983,9 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
                 pa.s_col = 4;
                 pa.s_blk = 0;
             }
-            const bool zp = h->Z != nullptr;
-            if (p.pf_rp == 0) e = launch_pf16(pa, zp, p.pf_ahead, p.grid_x, st);
-            else e = hp ? launch_pf4<true>(w.pf_attr, pa, zp, p.pf_rp, p.pf_ct, grid, st)
-                        : launch_pf4<false>(w.pf_attr, pa, zp, p.pf_rp, p.pf_ct, grid, st);
+            if (p.pf_rp == 0) e = launch_pf16(pa, p.pf_zp, p.pf_ahead, p.grid_x, st);
+            else e = hp ? launch_pf4<true>(w.pf_attr, pa, p.pf_zp, p.pf_rp, p.pf_ct, grid, st)
+                        : launch_pf4<false>(w.pf_attr, pa, p.pf_zp, p.pf_rp, p.pf_ct, grid, st);
         } else {
             PfArgs pa{};
             pa.W = reinterpret_cast<const char*>(h->W);
@@ -2489,8 +2497,9 @@ int i4_plan_query(int bits, int M, int K, int N, int flags, int n_cu, int32_t* o
     h.nblk = K / 32;
     h.nblk4 = (h.nblk + 3) / 4 * 4;
     h.nblk_pad = (h.nblk + JG - 1) / JG * JG;
-    h.extra = (flags & 32) != 0 || (flags & 64) != 0;
+    h.extra = (flags & (32 | 64 | 128)) != 0;
     h.has_dl = (flags & 64) != 0;
+    h.has_zp = bits == 4 && (flags & 128) != 0;
     h.has_ws = bits == 8;  // every INT8 handle carries its weight sums
     CallKind k;
     k.dots = (flags & 1) != 0;
@@ -2501,7 +2510,7 @@ int i4_plan_query(int bits, int M, int K, int N, int flags, int n_cu, int32_t* o
     k.tiles = N / 16;
     const Plan p = plan_call(h, M, k, n_cu);
     const int32_t v[] = {p.route, p.quant, p.fused, p.p64, p.lrec, p.rs, p.RG, p.NG, p.pair_xcd, p.lds,
-                         p.pf_rp, p.pf_ct, p.grid_x, p.grid_y, p.split, p.stream, p.flow};
+                         p.pf_rp, p.pf_ct, p.grid_x, p.grid_y, p.split, p.stream, p.flow, p.pf_ahead, p.pf_zp};
     const int n = std::min(nout, (int)(sizeof(v) / sizeof(v[0])));
     for (int i = 0; i < n; ++i) out[i] = v[i];
     return n;

@@ -835,7 +835,7 @@ __device__ inline T gload(gptr p) {
 struct Pf4Seg {
     const char* W;  // [tiles][nbg][64 lanes][16 B]
     const char* S;  // scales: of (tile t, column c, block j) at t s_tile + (4 (j / 4) >> sc_shift) s_grp + c s_col + (j & 3) s_blk
-    const char* Z;  // per-block zero points [tiles][nbg][16][4], or NULL (8 everywhere)
+    const char* Z;  // per-block zero points [tiles][nbg][16][4]; NULL, or unread, where all are 8
     float* C;       // [M][N]
     int N;
     int end;        // tiles of this and the segments before it (unused segments: INT_MAX)

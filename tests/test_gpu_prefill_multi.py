@@ -73,3 +73,28 @@ def test_mixed_layouts_still_run_one_by_one(gpu, hb, hi_prec):
     finally:
         hb.free(a)
         hb.free(b)
+
+
+@pytest.mark.parametrize("kernel", ["0", "1"])
+def test_zero_points_on_one_projection(gpu, hb, orc, hi_prec, monkeypatch, kernel):
+    """Per-block scales on both and explicit zero points on one: one device
+    layout, so one launch, which reads the zero points of both (8 on the one
+    without).  Equal bits to the oracle, in either order."""
+    K, N, M = 416, 80, 70
+    rng = np.random.default_rng(4)
+    w = [rng_weights(rng, N, K, 4, np.float32, z) for z in (False, True)]
+    hs = [hb.prepack(qw, sc, qz, K, N, bits=4) for qw, sc, qz in w]
+    monkeypatch.setenv("BREEZE_HIP_PF16", kernel)
+    A = rng.normal(size=(M, K)).astype(np.float32)
+    d = gpu.from_numpy(A).cuda()
+    try:
+        for hp in (True, False):
+            hb.set_hi_prec(hp)
+            want = [orc.matmul(qw, sc, qz, N, K, 4, A, hp) for qw, sc, qz in w]
+            for o in ((0, 1), (1, 0)):
+                got = hb.matmul_multi([hs[i] for i in o], d, [N, N])
+                for i, c in zip(o, got):
+                    assert bits_equal(c.cpu().numpy(), want[i]), (hp, o, i)
+    finally:
+        for h in hs:
+            hb.free(h)

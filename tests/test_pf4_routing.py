@@ -72,3 +72,14 @@ def test_every_output_is_covered(hb, M, N):
         assert p["grid_x"] * 4 >= N // 16 * -(-M // 16)
     else:
         assert p["grid_x"] * p["pf_ct"] >= N // 16 and p["grid_y"] * 32 * p["pf_rp"] >= M
+
+
+@pytest.mark.parametrize("M,N", [(33, 5120), (128, 17408)])
+def test_zero_points_are_read_only_where_given(hb, M, N):
+    """Per-block scales alone (extra) leave the zero points at 8: the kernels
+    without them.  INT8 weights have none."""
+    assert hb.plan(4, M, 5120, N)["pf_zp"] == 0
+    assert hb.plan(4, M, 5120, N, extra=True)["pf_zp"] == 0
+    assert hb.plan(4, M, 5120, N, zeros=True)["pf_zp"] == 1
+    assert hb.plan(4, M, 5120, N, pair=True, zeros=True)["pf_zp"] == 1
+    assert hb.plan(8, M, 5120, N, extra=True)["pf_zp"] == 0

@@ -336,12 +336,12 @@ QUANTIZERS = {0: None, 1: "staged", 2: "rows8", 3: "prefill"}
 
 
 def plan(bits, M, K, N, n_cu=256, dots=False, argmax=False, pair=False, multi=False, norm=False, extra=False,
-         legacy_corr=False, zeros=False):
+         legacy_corr=False, zeros=False, hi=True):
     """The library's routing decision for a call (i4_plan_query), without a
     device: which kernel, which stand-alone quantizer and the launch shape."""
     _require_lib()
     flags = (1 * dots) | (2 * argmax) | (4 * pair) | (8 * multi) | (16 * norm) | (32 * extra) | (64 * legacy_corr)
-    flags |= 128 * zeros
+    flags |= (128 * zeros) | (256 * (not hi))
     out = np.zeros(len(PLAN_FIELDS), np.int32)
     n = _lib.i4_plan_query(int(bits), int(M), int(K), int(N), flags, int(n_cu), _p(out), len(out))
     if n < 0:

@@ -1240,12 +1240,23 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //     200 rows as two launches of this kernel); RMSNorm + in_qkv/z/b/a at 33 /
 //     128 / 300 rows 247 / 283 / 345 -> 62 / 88 / 131; q/k/v 183 / 208 / 306 ->
 //     44 / 63 / 112.
-//   kPf4Start (0.6)  the workgroup shape of the rest (pick_pf4): a call takes
-//     about 40 us + 25 us a column group of the busiest wave at K=5120 (N=17408
-//     at 64 / 128 / 256 / 512 rows, shapes (2, 8) / (4, 8) / (4, 9) / (4, 17):
-//     61 / 82 / 104 / 162), and as much again for a second round; five tiles a
-//     workgroup leave half a group empty (N=17408 at 128 rows 84.7 against
-//     82.3 on eight, N=5120 at 512 rows 100 against 92).
+//   kPf4Costs, kPf16Cost4  the rest of the INT4 prefill takes the launch of
+//     least cost: 4.9 us, then per round of workgroups 1.7 us, 60 ns a row
+//     pair by column tile (the stores) and the shape's ns a block.  Zero
+//     points and the activation mode change a shape's ns a block by up to
+//     half, and K decides between them and the stores, so both are in it.
+//     Fitted to 13 shapes and the independent waves over K 512 to 12288, N
+//     1024 to 27648 and 33 to 1024 rows, both modes, with and without zero
+//     points: what it picks is 0.7% off the best on average, 12% at most
+//     (N=27648, 160 rows).  Against one cost for all, without five tiles:
+//     K=5120 N=17408 at 128 rows (eight tiles -> five) 84.2 -> 74.9, zero
+//     points 97.4 -> 83.2, INT8 activations with them 87.7 -> 73.1; K=1024
+//     26.1 -> 21.9; N=5120 400 rows, zero points 99.6 -> 86.6 (these with the
+//     kernel's stores and first loads as now); K=2048 N=5120 160 rows, INT8
+//     activations and zero points (independent waves -> (2, 4)) 31.3 -> 21.7.
+//     Two-pass calls without zero points keep the bounds drawn for them
+//     before: independent waves to 13 tiles a CU, four-wave shapes as if two
+//     a CU.
 //   kStreamIdleDiv (8)  plain decode calls read their weight chunks with
 //     non-temporal loads when at most one in 8 of a tile's producer slots
 //     (15 a phase) is idle.  Weights are read once a call; the hint streams
@@ -1306,7 +1317,6 @@ constexpr int kDec8LrecTiles = 2;
 constexpr int kPrefillMinRows = 9;
 constexpr int kSplitMaxTiles = 8, kSplitMinPhases = 20;
 constexpr int kPf16TilesPerCu = 13, kPf16TilesPerCu8 = 13, kPf16DeepPerCu = 6;
-constexpr double kPf4Start = 0.6;
 constexpr int kStreamIdleDiv = 8, kStreamMaxGroups = 2;
 
 // Row-blocks the decode prologue quantizes itself for calls of M rows
@@ -1406,6 +1416,7 @@ struct CallKind {
     bool pair = false;    // gate/up pair in one launch
     bool multi = false;   // several projections in one launch
     bool norm = false;    // multi with the RMSNorm in the prologue
+    bool hp = true;       // two-pass INT16 activations (false: INT8)
     int tiles = 0;        // column tiles of the launch (all segments of a multi call)
 };
 
@@ -1494,51 +1505,65 @@ int split_pieces(const Shape& h, int M, const CallKind& k, int n_cu, int* lds) {
     return S;
 }
 
-// Whether a prefill call of few output tiles a CU runs as independent 16-row
-// waves (see the routing table).  BREEZE_HIP_PF16=0 / 1 turns them off / on; a
-// forced workgroup shape turns them off.
-bool pick_pf16(Plan& p, int bits, int M, int tiles, int n_cu) {
-    const char* env = std::getenv("BREEZE_HIP_PF16");
-    const long waves = (long)tiles * ((M + 15) / 16);
-    const long most = (long)(bits == 4 ? kPf16TilesPerCu : kPf16TilesPerCu8) * n_cu;
-    const bool few = waves <= most && !std::getenv("BREEZE_HIP_PREFILL_RP") && !std::getenv("BREEZE_HIP_PREFILL_CT");
-    if (!(env ? env[0] == '1' : few)) return false;
-    p.pf_rp = 0;
-    p.pf_ct = 1;
-    p.pf_ahead = waves <= (long)kPf16DeepPerCu * n_cu ? 4 : 2;
-    p.grid_x = (int)((waves + kPf16Waves - 1) / kPf16Waves);
-    p.grid_y = 1;
-    return true;
+// What an INT4 prefill call takes by its launch, in ns (see the routing table).
+//
+// Independent 16-row waves: per workgroup of the busiest CU `start` ns and
+// `per` ns a block, besides `once` ns a block.
+struct Pf16Cost {
+    int start, once, per;
+};
+double pf16_cost(const Pf16Cost& c, int nblk, long waves, int n_cu) {
+    const long wgs = (waves + kPf16Waves - 1) / kPf16Waves, n = (wgs + n_cu - 1) / n_cu;
+    return 4550.0 + (double)(n * c.start) + nblk * (c.once + (double)(n * c.per));
 }
+// By (explicit zero points, four weight chunks in flight).
+constexpr Pf16Cost kPf16Cost4[2][2] = {{{550, 97, 57}, {550, 76, 47}}, {{800, 66, 80}, {800, 58, 74}}};
+// Workgroup shapes: ns a block of one round, for two-pass calls, two-pass with
+// zero points, INT8 activations, and those with zero points.  Shapes of four
+// waves run two workgroups a CU; `half` is for a single round of one.
+struct Pf4Cost {
+    int rp, ct, ns[4], half[4];
+};
+constexpr Pf4Cost kPf4Costs[] = {
+    {4, 17, {784, 1063, 679, 891}, {}}, {4, 16, {744, 964, 644, 832}, {}}, {4, 13, {655, 833, 576, 741}, {}},
+    {4, 12, {599, 747, 509, 657}, {}},  {4, 9, {500, 620, 417, 539}, {}},  {4, 8, {440, 531, 377, 463}, {}},
+    {4, 5, {381, 444, 326, 399}, {}},   {4, 4, {340, 370, 240, 300}, {}},  {2, 16, {467, 553, 391, 492}, {}},
+    {2, 8, {313, 357, 226, 292}, {}},   {2, 4, {380, 420, 283, 326}, {0, 250, 193, 235}},
+    {1, 16, {362, 417, 290, 328}, {}},  {1, 8, {356, 425, 307, 325}, {0, 264, 217, 241}},
+};
+static_assert(sizeof(kPf4Costs) / sizeof(kPf4Costs[0]) == kPfNumCfgs, "one cost per shape of kPfCfgs");
 
-// The INT4 prefill's workgroup shape: the one whose rounds x (half the column
-// groups of a CU's busiest SIMD + kPf4Start) is least; a CU holds eight waves.
+// Two-pass calls without explicit zero points keep the bounds drawn for them
+// before the costs were: independent waves up to kPf16TilesPerCu, and shapes
+// of four waves counted as filling their rounds.
+bool pf4_plain(const Shape& h, const CallKind& k) { return k.hp && !h.has_zp; }
+
+// The INT4 prefill's workgroup shape: the one of least cost.  Returns it.
 // BREEZE_HIP_PREFILL_RP / _CT force a shape.
-void pick_pf4(Plan& p, int M, int tiles, int n_cu) {
+double pick_pf4(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, int n_cu) {
     const char* frp = std::getenv("BREEZE_HIP_PREFILL_RP");
     const char* fct = std::getenv("BREEZE_HIP_PREFILL_CT");
     const int rp = frp ? std::atoi(frp) : 0, ct = fct ? std::atoi(fct) : 0;
     bool rp_ok = false, ct_ok = false;
-    for (const PfCfg& c : kPfCfgs) {
+    for (const Pf4Cost& c : kPf4Costs) {
         rp_ok = rp_ok || c.rp == rp;
-        ct_ok = ct_ok || ((!rp || c.rp == rp) && c.ct == ct && ct != 5);
+        ct_ok = ct_ok || ((!rp || c.rp == rp) && c.ct == ct);
     }
+    const int v = (k.hp ? 0 : 2) + (h.has_zp ? 1 : 0);
     double best = -1.0;
-    for (const PfCfg& c : kPfCfgs) {
+    for (const Pf4Cost& c : kPf4Costs) {
         if ((rp_ok && c.rp != rp) || (ct_ok && c.ct != ct)) continue;
-        if (c.ct == 5) continue;  // half of its third column group is empty: (4, 8) is faster wherever it fits
-        const int groups = (c.ct + 1) / 2, parts = std::min(groups, kPfWaves / c.rp), waves_wg = c.rp * parts;
-        const int per_cu = std::max(1, kPfWaves / waves_wg);
-        int simd = 0;  // column groups on the busiest SIMD of a CU
-        for (int sm = 0; sm < 4; ++sm) {
-            int n = 0;
-            for (int w = sm; w < waves_wg; w += 4) n += groups / parts + (w / c.rp < groups % parts);
-            simd = std::max(simd, n * per_cu);
-        }
+        const int parts = std::min((c.ct + 1) / 2, kPfWaves / c.rp);
+        int per_cu = kPfWaves / (c.rp * parts);
         const long gx = (tiles + c.ct - 1) / c.ct, gy = (M + 32 * c.rp - 1) / (32 * c.rp);
-        const long slots = (long)n_cu * per_cu;
-        const double cost = (double)((gx * gy + slots - 1) / slots) * (0.5 * simd + kPf4Start);
-        if (best < 0 || cost < best || (cost == best && c.rp == 2 && c.ct == 8)) {
+        int ns = c.ns[v];
+        if (per_cu > 1 && gx * gy <= n_cu && !pf4_plain(h, k)) {
+            per_cu = 1;
+            ns = c.half[v];
+        }
+        const long rounds = (gx * gy + (long)n_cu * per_cu - 1) / ((long)n_cu * per_cu);
+        const double cost = 4900.0 + (double)rounds * (1700 + 60 * c.rp * c.ct * per_cu + (double)h.nblk * ns);
+        if (best < 0 || cost < best) {
             best = cost;
             p.pf_rp = c.rp;
             p.pf_ct = c.ct;
@@ -1546,6 +1571,29 @@ void pick_pf4(Plan& p, int M, int tiles, int n_cu) {
             p.grid_y = (int)gy;
         }
     }
+    return best;
+}
+
+// Whether a prefill call of few output tiles a CU runs as independent 16-row
+// waves, given what INT4 workgroups would take (see the routing table).
+// BREEZE_HIP_PF16=0 / 1 turns them off / on; a forced workgroup shape turns
+// them off.
+bool pick_pf16(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, int n_cu, double wg_cost) {
+    const char* env = std::getenv("BREEZE_HIP_PF16");
+    const long waves = (long)tiles * ((M + 15) / 16);
+    const bool deep = waves <= (long)kPf16DeepPerCu * n_cu;
+    const long most = (long)(h.bits == 4 ? kPf16TilesPerCu : kPf16TilesPerCu8) * n_cu;
+    bool take = waves <= most && !std::getenv("BREEZE_HIP_PREFILL_RP") &&
+                !std::getenv("BREEZE_HIP_PREFILL_CT");
+    if (take && h.bits == 4 && !pf4_plain(h, k))
+        take = pf16_cost(kPf16Cost4[h.has_zp][deep], h.nblk, waves, n_cu) <= wg_cost;
+    if (!(env ? env[0] == '1' : take)) return false;
+    p.pf_rp = 0;
+    p.pf_ct = 1;
+    p.pf_ahead = deep ? 4 : 2;
+    p.grid_x = (int)((waves + kPf16Waves - 1) / kPf16Waves);
+    p.grid_y = 1;
+    return true;
 }
 
 Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
@@ -1576,7 +1624,7 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
         const int tiles = (k.tiles > 0 ? k.tiles : ntiles) * (k.pair ? 2 : 1);
         const int rows = 32 * pick_pf_rp(M, nullptr);
         p.Mpad = (M + rows - 1) / rows * rows;
-        if (!pick_pf16(p, h.bits, M, tiles, n_cu)) pick_pf4(p, M, tiles, n_cu);
+        pick_pf16(p, h, k, M, tiles, n_cu, pick_pf4(p, h, k, M, tiles, n_cu));
         return p;
     }
     int Mr_max = std::min(M, 4);
@@ -1622,11 +1670,11 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
         const int rows = 32 * p.pf_rp;
         p.Mpad = (M + rows - 1) / rows * rows;
         p.grid_y = p.Mpad / rows;
-        if (pick_pf16(p, h.bits, M, tiles, n_cu)) return p;
         if (h.bits == 4) {
-            pick_pf4(p, M, tiles, n_cu);
+            pick_pf16(p, h, k, M, tiles, n_cu, pick_pf4(p, h, k, M, tiles, n_cu));
             return p;
         }
+        if (pick_pf16(p, h, k, M, tiles, n_cu, 0.0)) return p;
         p.pf_ct = pick_pf_ct(tiles, p.grid_y, p.pf_rp, n_cu, std::getenv("BREEZE_HIP_PREFILL_CT"));
         p.grid_x = (tiles + p.pf_ct - 1) / p.pf_ct;
     } else if (dec8) {
@@ -1741,6 +1789,7 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
     kind.pair = h2 != nullptr;
     kind.multi = mp != nullptr;
     kind.norm = mp && mp->norm;
+    kind.hp = hp;
     kind.tiles = a.ntiles;
     if (mp) {
         kind.tiles = 0;
@@ -2507,6 +2556,7 @@ int i4_plan_query(int bits, int M, int K, int N, int flags, int n_cu, int32_t* o
     k.pair = (flags & 4) != 0;
     k.multi = (flags & 8) != 0;
     k.norm = (flags & 16) != 0;
+    k.hp = (flags & 256) == 0;
     k.tiles = N / 16;
     const Plan p = plan_call(h, M, k, n_cu);
     const int32_t v[] = {p.route, p.quant, p.fused, p.p64, p.lrec, p.rs, p.RG, p.NG, p.pair_xcd, p.lds,

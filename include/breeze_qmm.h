@@ -158,7 +158,7 @@ int i4_rmsnorm_matmul_multi_dev(const float* dX, const float* dNormW, float eps,
  * handle.  flags: 1 block-integer export, 2 argmax, 4 gate/up pair,
  * 8 multi-projection (one segment of N), 16 RMSNorm in that launch,
  * 32 per-block metadata (small scale groups), 64 legacy corr, 128 explicit
- * zero points; n_cu: compute units of the device.  out[0..18] = route
+ * zero points, 256 INT8 activations; n_cu: compute units of the device.  out[0..18] = route
  * (1 decode in four-row groups, 2 decode in eight-row groups, 3 prefill
  * GEMM, 4 rows kernel, 0 no single launch takes a paired or multi call),
  * stand-alone quantizer (0 none: the decode prologue quantizes, 1 staged

@@ -83,3 +83,48 @@ def test_zero_points_are_read_only_where_given(hb, M, N):
     assert hb.plan(4, M, 5120, N, zeros=True)["pf_zp"] == 1
     assert hb.plan(4, M, 5120, N, pair=True, zeros=True)["pf_zp"] == 1
     assert hb.plan(8, M, 5120, N, extra=True)["pf_zp"] == 0
+
+
+COSTS = [
+    # (M, K, N), call -> (row pairs, column tiles) of the launch; zeros: explicit
+    # zero points, hi: two-pass activations.  Five tiles a workgroup where they
+    # fill one round that eight would leave half empty, whatever K and the mode.
+    ((128, 5120, 17408), dict(), (4, 5)),
+    ((128, 5120, 17408), dict(zeros=True), (4, 5)),
+    ((128, 5120, 17408), dict(zeros=True, hi=False), (4, 5)),
+    ((100, 5120, 17408), dict(zeros=True), (4, 5)),
+    ((128, 1024, 17408), dict(), (4, 5)),
+    ((128, 2048, 17408), dict(zeros=True), (4, 5)),
+    ((400, 5120, 5120), dict(zeros=True), (4, 5)),
+    ((200, 5120, 10240), dict(zeros=True), (4, 5)),
+    # 12.5 output tiles a CU: independent waves only without zero points, two
+    # passes, where the bound of 13 stands.
+    ((320, 5120, 2560), dict(), (0, 1)),
+    ((320, 5120, 2560), dict(zeros=True, hi=False), (2, 4)),
+    ((160, 2048, 5120), dict(zeros=True, hi=False), (2, 4)),
+    # Fewer: independent waves in every mode.
+    ((64, 5120, 5120), dict(zeros=True), (0, 1)),
+    ((64, 5120, 5120), dict(hi=False), (0, 1)),
+    # The largest shapes are those that fill one round.
+    ((512, 5120, 17408), dict(zeros=True, hi=False), (4, 17)),
+    ((200, 5120, 17408), dict(zeros=True), (4, 9)),
+]
+
+
+@pytest.mark.parametrize("shape,call,want", COSTS, ids=[f"{c[0]}{c[1]}" for c in COSTS])
+def test_int4_launch_of_least_cost(hb, shape, call, want):
+    p = hb.plan(4, *shape, n_cu=256, **call)
+    assert (p["pf_rp"], p["pf_ct"]) == want, p
+
+
+@pytest.mark.parametrize("call", [dict(zeros=True), dict(hi=False), dict(zeros=True, hi=False),
+                                  dict(pair=True, zeros=True, hi=False)])
+@pytest.mark.parametrize("M", [33, 100, 320, 1000])
+@pytest.mark.parametrize("N", [16, 48, 2560, 17408, 27648])
+def test_every_output_is_covered_in_every_mode(hb, M, N, call):
+    p = hb.plan(4, M, 1024, N, **call)
+    tiles = N // 16 * (2 if call.get("pair") else 1)
+    if p["pf_rp"] == 0:
+        assert p["grid_x"] * 4 >= tiles * -(-M // 16)
+    else:
+        assert p["grid_x"] * p["pf_ct"] >= tiles and p["grid_y"] * 32 * p["pf_rp"] >= M

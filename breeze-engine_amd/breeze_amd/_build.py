@@ -13,7 +13,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(PKG), "csrc")
 # Host code and small kernels; the decode and prefill kernels, one unit per
 # (bits, activation mode) so the device passes run side by side.
-SOURCES = ["qmm.hip", "pf16_w4.hip", "pf16_w8.hip"] + [f"{k}_w{b}_{m}.hip" for k in ("dec", "pf") for b in (4, 8) for m in ("hp", "lp")]
+SOURCES = ["qmm.hip", "pf16_w4.hip", "pf16_w8.hip", "pf_w4_i8.hip"] + [f"{k}_w{b}_{m}.hip" for k in ("dec", "pf") for b in (4, 8) for m in ("hp", "lp")]
 LIB_NAME = "libbreeze_qmm.so"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

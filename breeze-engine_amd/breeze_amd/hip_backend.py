@@ -330,7 +330,7 @@ def matmul_silu_mul(gate, up, a2d, N):
 
 
 PLAN_FIELDS = ("route", "quant", "fused", "p64", "lrec", "rows_per_group", "row_groups", "tile_ranges", "pair_xcd",
-               "lds", "pf_rp", "pf_ct", "grid_x", "grid_y", "split", "stream", "flow", "pf_ahead", "pf_zp")
+               "lds", "pf_rp", "pf_ct", "grid_x", "grid_y", "split", "stream", "flow", "pf_ahead", "pf_zp", "pf_i8")
 ROUTES = {0: None, 1: "decode", 2: "decode8", 3: "prefill", 4: "rows"}
 QUANTIZERS = {0: None, 1: "staged", 2: "rows8", 3: "prefill"}
 

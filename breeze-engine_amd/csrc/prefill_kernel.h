@@ -1,15 +1,17 @@
-// prefill_kernel.h -- the INT8 prefill GEMM (rows past the decode kernel's) and its
-// launcher, instantiated per activation mode by pf_w8_{hp,lp}.hip.
+// prefill_kernel.h -- the prefill GEMM on the INT8 matrix instructions and its
+// launcher: INT8 weights (pf_w8_{hp,lp}.hip), and INT4 weights with explicit
+// zero points under INT8 activations (pf_w4_i8.hip).
 #pragma once
 
 #include "qmm_common.h"
 
 namespace bq {
 
-template <bool HP, int SCM, int CT, int RP, int S>
+template <int BITS, bool HP, int SCM, int CT, int RP, int S>
 __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
-    using L = PfLayout<CT, SCM, RP, S>;
+    using L = PfLayout<CT, SCM, BITS, RP, S>;
     static_assert(S == 2 || S == 3, "ring depth");
+    static_assert(BITS == 8 || (!HP && SCM == 2), "INT4: INT8 activations, per-block metadata");
     extern __shared__ __align__(16) char pf_lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -30,24 +32,52 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
     const int nst = (nch + kPfChunks - 1) / kPfChunks;
     const bool odd = a.nblk & 1;
 
-    // Shared part of a chunk: loads k < kWJ load weight tile
-    // min(wave + kPfWaves k, CT - 1) (a spare load repeats the last tile: same
-    // bytes, same place).  Loads k >= kWJ load the 1 KB of sums and scales at
-    // x0 = kWS + 1024 u, u = (k - kWJ) * kPfWaves + wave (clamped), lane bytes
-    // x0 + 16*lane.
+    // Shared part of a chunk (INT8) or stage (INT4).
+    // INT8: loads k < kWJ load weight tile min(wave + kPfWaves k, CT - 1)
+    // (a spare load repeats the last tile: same bytes, same place).  Loads
+    // k >= kWJ load the 1 KB of sums and scales at x0 = kWS + 1024 u,
+    // u = (k - kWJ) * kPfWaves + wave (clamped), lane bytes x0 + 16*lane.
+    // INT4: slot k loads unit u = k * kPfWaves + wave (clamped): raw tile u
+    // of the stage into chunk 0's weight area, or KB u - CT of the raw area.
     const char* src0[L::kPerWave];
     uint32_t step[L::kPerWave], gstep[L::kPerWave], x0s[L::kPerWave];
+    bool to_raw[L::kPerWave];
 #pragma unroll
     for (int k = 0; k < L::kPerWave; ++k) {
-        const int u = min((k - L::kWJ) * kPfWaves + wave, L::kSU - 1);
-        const int x0 = L::kWS + u * 1024;
+        const int u = BITS == 8 ? min((k - L::kWJ) * kPfWaves + wave, L::kSU - 1)
+                                : min(k * kPfWaves + wave, L::kUnits - 1);
+        const int x0 = BITS == 8 ? L::kWS + u * 1024 : u * 1024;
         const int x = x0 + 16 * lane;
         x0s[k] = (uint32_t)x0;
         gstep[k] = 0;
         step[k] = 0;
         src0[k] = a.W;
-        if (k < L::kWJ) continue;
-        if (x < L::kSB) {
+        to_raw[k] = false;
+        if (BITS == 8 && k < L::kWJ) continue;
+        if (BITS == 4) {
+            if (u < CT) {
+                const int tc = min(t0 + u, a.ntiles - 1);
+                src0[k] = a.W + (size_t)tc * a.nbg * 1024 + 16 * lane;
+                step[k] = 1024;
+                x0s[k] = (uint32_t)(u * 1024);
+            } else {
+                const int y = (u - CT) * 1024 + 16 * lane;
+                to_raw[k] = true;
+                x0s[k] = (uint32_t)((u - CT) * 1024);  // within the stage's raw area
+                src0[k] = a.S;  // padding lanes: any valid source
+                step[k] = 0;
+                if (y < L::kRawZ) {
+                    const int tc = min(t0 + (y >> 8), a.ntiles - 1);
+                    src0[k] = a.S + (size_t)tc * a.nbg * 256 + (y & 255);
+                    step[k] = 256;
+                } else if (y < L::kRawUsed) {
+                    const int yz = y - L::kRawZ;
+                    const int tc = min(t0 + (yz >> 6), a.ntiles - 1);
+                    src0[k] = a.Z + (size_t)tc * a.nbg * 64 + (yz & 63);
+                    step[k] = 64;
+                }
+            }
+        } else if (x < L::kSB) {
             const int y = x - L::kWS;
             const int tc = min(t0 + (y >> 7), a.ntiles - 1);
             src0[k] = a.WS + (size_t)tc * nch * 128 + (y & 127);
@@ -83,27 +113,33 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
     // Load d of this wave's kDmaChunk loads of chunk c into the chunk region
     // at LDS address cbase: the shared slots, then its record units.
     constexpr int kDmaChunk = L::kPerWave + kRecPerWave;
-    auto dma_slot = [&](int c, uint32_t cbase, int d) __attribute__((always_inline)) {
+    // INT4: only chunk 0 of a stage (first) carries the stage's shared loads;
+    // raw is the LDS address of the stage's raw area.
+    auto dma_slot = [&](int c, uint32_t cbase, int d, bool first, uint32_t raw) __attribute__((always_inline)) {
         if (d < L::kPerWave) {
-            if (d < L::kWJ) {
+            if (BITS == 8 && d < L::kWJ) {
                 const int tile = min(d * kPfWaves + wave, CT - 1);
                 const int tc = min(t0 + tile, a.ntiles - 1);
                 dma16s(a.W + ((size_t)tc * nch + c) * 1024, 16 * lane, cbase + (uint32_t)(tile * 1024));
-            } else {
+            } else if (BITS == 8) {
                 const size_t g = SCM == 1 ? (size_t)((2 * c) >> a.sc_shift) : 0;
                 dma16(src0[d] + (size_t)c * step[d] + g * gstep[d], cbase + x0s[d]);
+            } else if (first) {
+                dma16(src0[d] + (size_t)(c >> 1) * step[d], (to_raw[d] ? raw : cbase) + x0s[d]);
             }
         } else {
             const int e = d - L::kPerWave;
             dma16s(rec0 + rec_src[e] + (size_t)c * kRecBytes, 16 * lane, cbase + rec_dst[e]);
         }
     };
+    // Raw area of stage g (INT4).
+    auto raw_base = [&](int g) { return lds0 + (uint32_t)(L::kRawOff + (g % L::kNRaw) * L::kRaw); };
     // With more than two stages every stage issues the same loads per wave
     // (chunks past the end repeat the last chunk's, into a slot nobody
     // reads), so the wait at a stage's start counts the loads issued after
     // it exactly.  Two stages wait for all loads and skip those chunks (the
     // loads kept the allocator from fitting the widest shapes' registers).
-    constexpr int kStageLoads = kPfChunks * kDmaChunk;
+    constexpr int kStageLoads = BITS == 8 ? kPfChunks * kDmaChunk : kDmaChunk + (kPfChunks - 1) * kRecPerWave;
     auto issue_stage = [&](int g, int buf) __attribute__((always_inline)) {
         const uint32_t sbase = lds0 + (uint32_t)(buf * L::kStage);
 #pragma unroll
@@ -111,7 +147,57 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
             const int c = min(g * kPfChunks + cc, nch - 1);
             if (S == 2 && g * kPfChunks + cc >= nch) continue;
 #pragma unroll
-            for (int d = 0; d < kDmaChunk; ++d) dma_slot(c, sbase + (uint32_t)(cc * L::kChunk), d);
+            for (int d = 0; d < kDmaChunk; ++d) dma_slot(c, sbase + (uint32_t)(cc * L::kChunk), d, cc == 0, raw_base(g));
+        }
+    };
+
+    // INT4: expands stage g (buffer buf) in place from its raw area (with more
+    // than one row pair all threads share the tiles and a workgroup barrier
+    // must follow).  Wave w takes tiles w, w + 8, ... (with one row pair, the
+    // tiles of its column part); each lane takes one (column, k-octet) of
+    // the tile and writes that octet of the four blocks where pf_w_byte puts
+    // it.
+    auto expand = [&](int g, int buf) {
+        if constexpr (BITS == 4) {
+            char* sb = pf_lds + buf * L::kStage;
+            const char* raw = pf_lds + L::kRawOff + (g % L::kNRaw) * L::kRaw;
+            // Lane l expands octet o of column c of the tile, with
+            // c = (l & 7) + 8 ((l >> 4) & 1) and o = ((l >> 3) & 1) + 2 (l >> 5):
+            // eight lanes read 128 contiguous raw bytes, and sixteen lanes
+            // write 128 contiguous bytes of operands (pf_w_byte), so neither
+            // side has bank conflicts.
+            const int c = (lane & 7) + 8 * ((lane >> 4) & 1), o = ((lane >> 3) & 1) + 2 * (lane >> 5);
+            // One row pair: each wave expands the tiles of its own column
+            // part, which no other wave reads, so no barrier has to follow.
+            const int t_beg = RP == 1 ? part_t0 : wave, t_end = RP == 1 ? part_t0 + part_nt : CT;
+            const int t_step = RP == 1 ? 1 : kPfWaves;
+            for (int t = t_beg; t < t_end; t += t_step) {
+                const uint4 w = *reinterpret_cast<const uint4*>(sb + t * 1024 + 16 * (c + 16 * o));
+                const uint32_t z = *reinterpret_cast<const uint32_t*>(raw + L::kRawZ + t * 64 + 4 * c);
+                const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
+                // Octet o of blocks 0-3 (chunk b >> 1, block b & 1) into the
+                // operand order; this wave alone reads and writes tile t,
+                // and all of its reads of t are done (the writes use them).
+                uint32_t lo[4], hi[4];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    // b = n - zp as a signed byte: n + (128 - zp), then flip
+                    // the top bit.  zp is a signed byte in [-112, 127]
+                    // (i4_prepack sends lower legacy zero points to the INT8
+                    // representation), so 128 - zp is in [1, 240] and
+                    // n + 128 - zp in [1, 255]: no carry crosses a byte.
+                    const uint32_t zr = (uint32_t)(128 - (int)(int8_t)(z >> (8 * b))) * 0x01010101u;
+                    lo[b] = ((wv[b] & 0x0F0F0F0Fu) + zr) ^ 0x80808080u;
+                    hi[b] = (((wv[b] >> 4) & 0x0F0F0F0Fu) + zr) ^ 0x80808080u;
+                }
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    *reinterpret_cast<uint2*>(sb + (b >> 1) * L::kChunk + t * 1024 + pf_w_byte(4, c, o, b & 1)) =
+                        make_uint2(lo[b], hi[b]);
+                if (o < 2)  // the scales of chunk o's two blocks
+                    *reinterpret_cast<float2*>(sb + o * L::kChunk + L::kSB + t * 128 + 8 * c) =
+                        *reinterpret_cast<const float2*>(raw + t * 256 + 16 * c + 8 * o);
+            }
         }
     };
 
@@ -126,8 +212,9 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
     // acc = fma(s_a, f32(cs) * s_b, acc) in block order.
     // Lane l: A row / output column c32 = l & 31, k half kh = l >> 5.  The A
     // operand is one 16-byte LDS read: records hold k-octets 2 kh and
-    // 2 kh + 1 of a row side by side (pf_rec_byte).  Weight tiles hold octet o
-    // of both blocks side by side, and B takes two 8-byte halves 256 bytes apart (pf_w_byte).  Reading those
+    // 2 kh + 1 of a row side by side (pf_rec_byte).  So do expanded INT4
+    // tiles for B; INT8 tiles hold octet o of both blocks side by side, and
+    // B takes two 8-byte halves 256 bytes apart (pf_w_byte).  Reading those
     // with one ds_read2_b64 straight into the operand was slower than the
     // register moves after a merged 16-byte read: an 8-byte access at a
     // 16-byte lane stride uses half the LDS banks.
@@ -162,11 +249,13 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
             for (int i = 0; i < 4; ++i) acco[r][i] = 0.0f;
 
         // dma_tag: 0 no loads, 1 or 2 the loads of chunk 0 or 1 of the stage
-        // S - 1 ahead (chunk c_next, at LDS nbase).
-        auto compute = [&](const char* cp, auto nb_tag, auto dma_tag, int c_next, uint32_t nbase) {
+        // S - 1 ahead (chunk c_next, at LDS nbase; nraw: that buffer's raw
+        // area).
+        auto compute = [&](const char* cp, auto nb_tag, auto dma_tag, int c_next, uint32_t nbase, uint32_t nraw) {
             constexpr int NB = decltype(nb_tag)::value;
             constexpr bool DMA = decltype(dma_tag)::value != 0;
             constexpr bool BOTH = decltype(dma_tag)::value == 3;  // both chunks of the next stage
+            constexpr bool FIRST = decltype(dma_tag)::value == 1 || BOTH;
             const int c_next2 = min(c_next + 1, nch - 1);
             constexpr int kAhead = 1;            // groups read ahead
             constexpr int NGB = NG * NB;         // group steps
@@ -215,7 +304,7 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
                 const int t = toff + CTW - 1;
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
-                    bwo[b] = *reinterpret_cast<const uint64_t*>(cp + t * 1024 + pf_w_byte(col, grp, b));
+                    bwo[b] = *reinterpret_cast<const uint64_t*>(cp + t * 1024 + pf_w_byte(BITS, col, grp, b));
                 if (HP) wso = *reinterpret_cast<const int2*>(cp + L::kWS + t * 128 + 8 * col);
                 if (SCM == 2) {
                     const float2 f = *reinterpret_cast<const float2*>(cp + L::kSB + t * 128 + 8 * col);
@@ -235,10 +324,14 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
                 const int t = toff + 2 * g + (c32 >> 4);
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
-                    const char* bp = cp + t * 1024 + pf_w_byte(c32 & 15, 2 * kh, b);
-                    const uint2 lo = *reinterpret_cast<const uint2*>(bp);
-                    const uint2 hi = *reinterpret_cast<const uint2*>(bp + 256);
-                    bq[g][b] = v4i{(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
+                    if (BITS == 8) {
+                        const char* bp = cp + t * 1024 + pf_w_byte(8, c32 & 15, 2 * kh, b);
+                        const uint2 lo = *reinterpret_cast<const uint2*>(bp);
+                        const uint2 hi = *reinterpret_cast<const uint2*>(bp + 256);
+                        bq[g][b] = v4i{(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
+                    } else {
+                        bq[g][b] = *reinterpret_cast<const v4i*>(cp + t * 1024 + pf_w_byte(4, c32 & 15, 2 * kh, b));
+                    }
                 }
                 if (HP) wsg[g] = *reinterpret_cast<const int2*>(cp + L::kWS + t * 128 + 8 * (c32 & 15));
                 if (SCM == 2) {
@@ -327,8 +420,8 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
 #pragma unroll
                 for (int e = 0; e < TL; ++e) {
                     if (e * NS / TL != s) continue;
-                    if (e < kDmaChunk) dma_slot(c_next, nbase, e);
-                    else dma_slot(c_next2, nbase + (uint32_t)L::kChunk, e - kDmaChunk);
+                    if (e < kDmaChunk) dma_slot(c_next, nbase, e, FIRST, nraw);
+                    else dma_slot(c_next2, nbase + (uint32_t)L::kChunk, e - kDmaChunk, false, nraw);
                 }
                 step_h(s + 1);
                 step_e(s);
@@ -358,6 +451,11 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
             else __builtin_amdgcn_s_waitcnt(vm_wait(0));
             lds_barrier();
             const int buf = g % S;
+            if (BITS == 4) {
+                expand(g, buf);
+                if (RP > 1) lds_barrier();
+                else asm volatile("" ::: "memory");
+            }
             const int gn = g + S - 1, bn = gn % S;  // stage issued now, and its buffer
             const uint32_t nbase = lds0 + (uint32_t)(bn * L::kStage);
             const int cn = min(gn * kPfChunks, nch - 1);
@@ -369,35 +467,41 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
                     if (S == 2) {
                         // Both chunks' loads during the first chunk: the
                         // second chunk's have a whole chunk to land.
-                        compute(sp, two, dma01, cn, nbase);
-                        compute(sp + L::kChunk, two, no_dma, 0, 0u);
+                        compute(sp, two, dma01, cn, nbase, raw_base(gn));
+                        compute(sp + L::kChunk, two, no_dma, 0, 0u, 0u);
                     } else {
-                        compute(sp, two, dma0, cn, nbase);
-                        compute(sp + L::kChunk, two, dma1, min(cn + 1, nch - 1), nbase + (uint32_t)L::kChunk);
+                        compute(sp, two, dma0, cn, nbase, raw_base(gn));
+                        compute(sp + L::kChunk, two, dma1, min(cn + 1, nch - 1), nbase + (uint32_t)L::kChunk,
+                                raw_base(gn));
                     }
                 } else {
                     issue_stage(gn, bn);
                 }
             } else if (S > 2 && active) {
                 const char* sp = pf_lds + buf * L::kStage;
-                compute(sp, two, no_dma, 0, 0u);
-                compute(sp + L::kChunk, two, no_dma, 0, 0u);
+                compute(sp, two, no_dma, 0, 0u, 0u);
+                compute(sp + L::kChunk, two, no_dma, 0, 0u, 0u);
             }
         }
         __builtin_amdgcn_s_waitcnt(vm_wait(0));
         lds_barrier();
+        if (BITS == 4) {
+            expand(nst - 1, (nst - 1) % S);
+            if (RP > 1) lds_barrier();
+            else asm volatile("" ::: "memory");
+        }
         if (!active) return;
         {
             const char* sp = pf_lds + ((nst - 1) % S) * L::kStage;
             const int c0 = (nst - 1) * kPfChunks;
             if (c0 + 1 < nch) {
-                compute(sp, two, no_dma, 0, 0u);
-                if (odd) compute(sp + L::kChunk, one, no_dma, 0, 0u);
-                else compute(sp + L::kChunk, two, no_dma, 0, 0u);
+                compute(sp, two, no_dma, 0, 0u, 0u);
+                if (odd) compute(sp + L::kChunk, one, no_dma, 0, 0u, 0u);
+                else compute(sp + L::kChunk, two, no_dma, 0, 0u, 0u);
             } else if (odd) {
-                compute(sp, one, no_dma, 0, 0u);
+                compute(sp, one, no_dma, 0, 0u, 0u);
             } else {
-                compute(sp, two, no_dma, 0, 0u);
+                compute(sp, two, no_dma, 0, 0u, 0u);
             }
         }
 #pragma unroll
@@ -433,13 +537,13 @@ __global__ __launch_bounds__(kPfWaves * 64) void prefill_kernel(PfArgs a) {
 }
 
 
-template <bool HP, int SCM, int CT, int RP, int S>
+template <int BITS, bool HP, int SCM, int CT, int RP, int S>
 hipError_t launch_pf_t(bool* pf_attr, const PfArgs& p, dim3 grid, hipStream_t st) {
-    using L = PfLayout<CT, SCM, RP, S>;
-    auto kern = prefill_kernel<HP, SCM, CT, RP, S>;
+    using L = PfLayout<CT, SCM, BITS, RP, S>;
+    auto kern = prefill_kernel<BITS, HP, SCM, CT, RP, S>;
     int slot = 0;
     while (kPfCfgs[slot].rp != RP || kPfCfgs[slot].ct != CT) ++slot;
-    const int key = (HP ? 1 : 0) | SCM << 1 | slot << 3;
+    const int key = (HP ? 1 : 0) | SCM << 1 | slot << 3 | (BITS == 4 ? 256 : 0);  // 128: pf4_kernel
     if (!pf_attr[key]) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, L::kBytes);
@@ -451,31 +555,35 @@ hipError_t launch_pf_t(bool* pf_attr, const PfArgs& p, dim3 grid, hipStream_t st
 }
 
 // One case per entry of kPfCfgs (row pairs, column tiles, ring stages).
-template <bool HP, int SCM>
+template <int BITS, bool HP, int SCM>
 hipError_t launch_pf_scm(bool* pf_attr, const PfArgs& p, int rp, int ct, dim3 grid, hipStream_t st) {
     switch (rp * 100 + ct) {
-        case 417: return launch_pf_t<HP, SCM, 17, 4, 2>(pf_attr, p, grid, st);
-        case 416: return launch_pf_t<HP, SCM, 16, 4, 2>(pf_attr, p, grid, st);
-        case 413: return launch_pf_t<HP, SCM, 13, 4, 2>(pf_attr, p, grid, st);
-        case 412: return launch_pf_t<HP, SCM, 12, 4, 2>(pf_attr, p, grid, st);
-        case 409: return launch_pf_t<HP, SCM, 9, 4, 2>(pf_attr, p, grid, st);
-        case 408: return launch_pf_t<HP, SCM, 8, 4, 2>(pf_attr, p, grid, st);
-        case 405: return launch_pf_t<HP, SCM, 5, 4, 2>(pf_attr, p, grid, st);
-        case 404: return launch_pf_t<HP, SCM, 4, 4, 2>(pf_attr, p, grid, st);
-        case 216: return launch_pf_t<HP, SCM, 16, 2, 2>(pf_attr, p, grid, st);
-        case 208: return launch_pf_t<HP, SCM, 8, 2, 3>(pf_attr, p, grid, st);
-        case 204: return launch_pf_t<HP, SCM, 4, 2, 3>(pf_attr, p, grid, st);
-        case 116: return launch_pf_t<HP, SCM, 16, 1, 2>(pf_attr, p, grid, st);
-        case 108: return launch_pf_t<HP, SCM, 8, 1, 3>(pf_attr, p, grid, st);
+        case 417: return launch_pf_t<BITS, HP, SCM, 17, 4, 2>(pf_attr, p, grid, st);
+        case 416: return launch_pf_t<BITS, HP, SCM, 16, 4, 2>(pf_attr, p, grid, st);
+        case 413: return launch_pf_t<BITS, HP, SCM, 13, 4, 2>(pf_attr, p, grid, st);
+        case 412: return launch_pf_t<BITS, HP, SCM, 12, 4, 2>(pf_attr, p, grid, st);
+        case 409: return launch_pf_t<BITS, HP, SCM, 9, 4, 2>(pf_attr, p, grid, st);
+        case 408: return launch_pf_t<BITS, HP, SCM, 8, 4, 2>(pf_attr, p, grid, st);
+        case 405: return launch_pf_t<BITS, HP, SCM, 5, 4, 2>(pf_attr, p, grid, st);
+        case 404: return launch_pf_t<BITS, HP, SCM, 4, 4, 2>(pf_attr, p, grid, st);
+        case 216: return launch_pf_t<BITS, HP, SCM, 16, 2, 2>(pf_attr, p, grid, st);
+        case 208: return launch_pf_t<BITS, HP, SCM, 8, 2, 3>(pf_attr, p, grid, st);
+        case 204: return launch_pf_t<BITS, HP, SCM, 4, 2, 3>(pf_attr, p, grid, st);
+        case 116: return launch_pf_t<BITS, HP, SCM, 16, 1, 2>(pf_attr, p, grid, st);
+        case 108: return launch_pf_t<BITS, HP, SCM, 8, 1, 3>(pf_attr, p, grid, st);
         default: return hipErrorInvalidValue;
     }
 }
 
-template <bool HP>
+template <int BITS, bool HP>
 hipError_t launch_pf(bool* pf_attr, const PfArgs& p, int scm, int rp, int ct, dim3 grid, hipStream_t st) {
-    if (scm == 2) return launch_pf_scm<HP, 2>(pf_attr, p, rp, ct, grid, st);
-    if (scm == 1) return launch_pf_scm<HP, 1>(pf_attr, p, rp, ct, grid, st);
-    return launch_pf_scm<HP, 0>(pf_attr, p, rp, ct, grid, st);
+    if constexpr (BITS == 4) {
+        return scm == 2 ? launch_pf_scm<4, HP, 2>(pf_attr, p, rp, ct, grid, st) : hipErrorInvalidValue;
+    } else {
+        if (scm == 2) return launch_pf_scm<8, HP, 2>(pf_attr, p, rp, ct, grid, st);
+        if (scm == 1) return launch_pf_scm<8, HP, 1>(pf_attr, p, rp, ct, grid, st);
+        return launch_pf_scm<8, HP, 0>(pf_attr, p, rp, ct, grid, st);
+    }
 }
 
 }  // namespace bq

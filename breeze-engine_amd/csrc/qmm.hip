@@ -434,9 +434,9 @@ int pick_pf_rp(int M, const char* force) {
 // Column tiles per workgroup for rp row pairs: among the instantiated
 // widths, the one that minimizes (workgroup rounds at one workgroup per CU)
 // x (tiles on the busiest SIMD, whose two waves hold column parts s / rp and
-// (s + 4) / rp).  `force` (BREEZE_HIP_PREFILL_CT) selects an instantiated
-// width for rp instead, for tests and tuning.
-int pick_pf_ct(int ntiles, int gy, int rp, int n_cu, const char* force) {
+// (s + 4) / rp); *rounds receives the rounds.  `force` (BREEZE_HIP_PREFILL_CT)
+// selects an instantiated width for rp instead, for tests and tuning.
+int pick_pf_ct(int ntiles, int gy, int rp, int n_cu, const char* force, int* rounds) {
     if (force) {
         const int v = std::atoi(force);
         for (const PfCfg& c : kPfCfgs)
@@ -457,6 +457,7 @@ int pick_pf_ct(int ntiles, int gy, int rp, int n_cu, const char* force) {
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
             best = c.ct;
+            *rounds = (int)((wgs + n_cu - 1) / n_cu);
         }
     }
     return best;
@@ -878,7 +879,7 @@ struct Workspace {
     int n_cu = 0;
     bool attr_set[1024] = {};  // decode kernel variants with the kernel attribute set
     bool dec8_attr[64] = {};  // the same for dec8_kernel, per (bits, mode) and (FUSE mode, metadata, LDS records)
-    bool pf_attr[256] = {};
+    bool pf_attr[384] = {};
 };
 
 constexpr int kMaxDevices = 64;
@@ -1257,6 +1258,16 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //     Two-pass calls without zero points keep the bounds drawn for them
 //     before: independent waves to 13 tiles a CU, four-wave shapes as if two
 //     a CU.
+//   Pf4Cost::i8  one projection past 64 rows with explicit zero points under
+//     INT8 activations compares its FP6 launch with workgroups on the INT8
+//     matrix instructions (nibble - zp in bytes): one digit there as here, and
+//     no zero-point FMA, 48 vector instructions a step on both, but the rows
+//     come through LDS and the stores and the first stage cost 2 us a round
+//     less.  FP6 -> INT8: K=5120 N=17408 at 128 / 512 rows 78.7 -> 71 / 160.6 ->
+//     148, K=1024 N=17408 1024 rows 80.9 -> 71.4, N=5120 400 rows 22.0 ->
+//     20.3; FP6 stays where a shape fits better (K=5120 N=2560, 320 rows: 47
+//     against 61).  Over K 512 to 12288 and N 1024 to 27648 the pick is 0.5%
+//     off the better one on average.
 //   kStreamIdleDiv (8)  plain decode calls read their weight chunks with
 //     non-temporal loads when at most one in 8 of a tile's producer slots
 //     (15 a phase) is idle.  Weights are read once a call; the hint streams
@@ -1304,7 +1315,8 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 // every prologue-quantized call), BREEZE_HIP_DEC8_ROWS (their row limit),
 // BREEZE_HIP_DEC8_LREC (0: records never in LDS; n: from n tiles),
 // BREEZE_HIP_PREFILL_RP / _CT (prefill workgroup shape), BREEZE_HIP_PF16 (the
-// prefill's independent waves: 0 never, 1 always), BREEZE_HIP_FUSED_MAX_BLOCKS
+// prefill's independent waves: 0 never, 1 always), BREEZE_HIP_PF_I8 (INT4
+// prefill on the INT8 instructions: 0 never, 1 where it can), BREEZE_HIP_FUSED_MAX_BLOCKS
 // (row-blocks the decode prologue quantizes), BREEZE_HIP_SPLIT (split-K),
 // BREEZE_HIP_STREAM (non-temporal weight loads), BREEZE_HIP_FLOW (phases
 // across tile boundaries).
@@ -1434,6 +1446,7 @@ struct Plan {
     // rows, weight chunks in flight of the independent waves.
     int pf_rp = 0, pf_ct = 0, Mpad = 0, pf_ahead = 0;
     bool pf_zp = false;      // INT4 prefill: the kernel reads zero points
+    bool pf_i8 = false;      // INT4 prefill on the INT8 matrix instructions
     int grid_x = 0, grid_y = 1;
     int split = 0;           // decode split-K: workgroups per tile (0: none)
     bool stream = false;     // decode: weight chunks read with non-temporal loads
@@ -1520,16 +1533,19 @@ double pf16_cost(const Pf16Cost& c, int nblk, long waves, int n_cu) {
 constexpr Pf16Cost kPf16Cost4[2][2] = {{{550, 97, 57}, {550, 76, 47}}, {{800, 66, 80}, {800, 58, 74}}};
 // Workgroup shapes: ns a block of one round, for two-pass calls, two-pass with
 // zero points, INT8 activations, and those with zero points.  Shapes of four
-// waves run two workgroups a CU; `half` is for a single round of one.
+// waves run two workgroups a CU; `half` is for a single round of one.  `i8`:
+// the same shape on the INT8 matrix instructions (pf4_i8).
 struct Pf4Cost {
-    int rp, ct, ns[4], half[4];
+    int rp, ct, ns[4], half[4], i8;
 };
 constexpr Pf4Cost kPf4Costs[] = {
-    {4, 17, {784, 1063, 679, 891}, {}}, {4, 16, {744, 964, 644, 832}, {}}, {4, 13, {655, 833, 576, 741}, {}},
-    {4, 12, {599, 747, 509, 657}, {}},  {4, 9, {500, 620, 417, 539}, {}},  {4, 8, {440, 531, 377, 463}, {}},
-    {4, 5, {381, 444, 326, 399}, {}},   {4, 4, {340, 370, 240, 300}, {}},  {2, 16, {467, 553, 391, 492}, {}},
-    {2, 8, {313, 357, 226, 292}, {}},   {2, 4, {380, 420, 283, 326}, {0, 250, 193, 235}},
-    {1, 16, {362, 417, 290, 328}, {}},  {1, 8, {356, 425, 307, 325}, {0, 264, 217, 241}},
+    {4, 17, {784, 1063, 679, 891}, {}, 861}, {4, 16, {744, 964, 644, 832}, {}, 830},
+    {4, 13, {655, 833, 576, 741}, {}, 705},  {4, 12, {599, 747, 509, 657}, {}, 642},
+    {4, 9, {500, 620, 417, 539}, {}, 546},   {4, 8, {440, 531, 377, 463}, {}, 458},
+    {4, 5, {381, 444, 326, 399}, {}, 380},   {4, 4, {340, 370, 240, 300}, {}, 308},
+    {2, 16, {467, 553, 391, 492}, {}, 0},    {2, 8, {313, 357, 226, 292}, {}, 0},
+    {2, 4, {380, 420, 283, 326}, {0, 250, 193, 235}, 0},
+    {1, 16, {362, 417, 290, 328}, {}, 0},    {1, 8, {356, 425, 307, 325}, {0, 264, 217, 241}, 0},
 };
 static_assert(sizeof(kPf4Costs) / sizeof(kPf4Costs[0]) == kPfNumCfgs, "one cost per shape of kPfCfgs");
 
@@ -1574,6 +1590,24 @@ double pick_pf4(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, in
     return best;
 }
 
+// The INT8 matrix instructions' workgroups (prefill_kernel) of 128 rows by ct
+// tiles for INT4 weights, in rounds of one a CU.
+double pf4_i8_cost(int nblk, int rounds, int ct) {
+    int ns = 0;
+    for (const Pf4Cost& c : kPf4Costs)
+        if (c.rp == 4 && c.ct == ct) ns = c.i8;
+    return 3100.0 + (double)rounds * (1300 + 334 * ct + (double)nblk * ns);
+}
+// Whether an INT4 prefill call that could take them (explicit zero points
+// under INT8 activations, one projection) does (see the routing table).
+// BREEZE_HIP_PF_I8=0 / 1 turns them off / on; a forced workgroup shape turns
+// them off.
+bool take_pf4_i8(const Shape& h, const CallKind& k, int M, double cost, double fp6_cost) {
+    if (k.hp || !h.has_zp) return false;
+    if (const char* env = std::getenv("BREEZE_HIP_PF_I8")) return env[0] == '1';
+    return M > 64 && cost < fp6_cost && !std::getenv("BREEZE_HIP_PREFILL_RP") && !std::getenv("BREEZE_HIP_PREFILL_CT");
+}
+
 // Whether a prefill call of few output tiles a CU runs as independent 16-row
 // waves, given what INT4 workgroups would take (see the routing table).
 // BREEZE_HIP_PF16=0 / 1 turns them off / on; a forced workgroup shape turns
@@ -1590,6 +1624,7 @@ bool pick_pf16(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, int
     if (!(env ? env[0] == '1' : take)) return false;
     p.pf_rp = 0;
     p.pf_ct = 1;
+    p.pf_i8 = false;
     p.pf_ahead = deep ? 4 : 2;
     p.grid_x = (int)((waves + kPf16Waves - 1) / kPf16Waves);
     p.grid_y = 1;
@@ -1670,12 +1705,24 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
         const int rows = 32 * p.pf_rp;
         p.Mpad = (M + rows - 1) / rows * rows;
         p.grid_y = p.Mpad / rows;
+        int rounds = 1;
+        const int ct = pick_pf_ct(tiles, p.grid_y, p.pf_rp, n_cu, std::getenv("BREEZE_HIP_PREFILL_CT"), &rounds);
         if (h.bits == 4) {
-            pick_pf16(p, h, k, M, tiles, n_cu, pick_pf4(p, h, k, M, tiles, n_cu));
+            Plan i8 = p;
+            i8.pf_i8 = true;
+            i8.pf_ct = ct;
+            i8.grid_x = (tiles + ct - 1) / ct;
+            double cost = pick_pf4(p, h, k, M, tiles, n_cu);
+            const double c8 = pf4_i8_cost(h.nblk, rounds, ct);
+            if (take_pf4_i8(h, k, M, c8, cost)) {
+                p = i8;
+                cost = c8;
+            }
+            pick_pf16(p, h, k, M, tiles, n_cu, cost);
             return p;
         }
         if (pick_pf16(p, h, k, M, tiles, n_cu, 0.0)) return p;
-        p.pf_ct = pick_pf_ct(tiles, p.grid_y, p.pf_rp, n_cu, std::getenv("BREEZE_HIP_PREFILL_CT"));
+        p.pf_ct = ct;
         p.grid_x = (tiles + p.pf_ct - 1) / p.pf_ct;
     } else if (dec8) {
         p.route = kRouteDec8;
@@ -1816,7 +1863,7 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
         // Records in MFMA operand order for the prefill GEMM.
         const int nch_rec = (h->nblk + 1) / 2;  // record chunks of two blocks
         const size_t int8_bytes = (size_t)(p.Mpad / 16) * nch_rec * kRecBytes;
-        if (h->bits == 4) {
+        if (h->bits == 4 && !p.pf_i8) {
             const int rtiles = (M + 31) / 32 * 2, mult = p.pf_zp ? 1 : 8;
             // The fixed scratch counts the INT8 records' bytes (the array is
             // larger by the FP6 records' share, kNoAllocArray).
@@ -1826,7 +1873,7 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
             const unsigned qb = (unsigned)((waves + 3) / 4);
             if (hp) quantize_f6_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, rtiles, mult, s.rec);
             else quantize_f6_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, rtiles, mult, s.rec);
-        } else if (p.pf_rp == 0) {
+        } else if (p.pf_rp == 0) {  // INT8 weights
             const int rtiles = (M + 15) / 16;
             const size_t bytes = s.fixed ? int8_bytes : (size_t)rtiles * nch_rec * r16_rec_bytes(hp);
             if (!grow(w, st, &s.rec, &s.rec_cap, bytes, "workspace alloc", s.fixed)) return -4;
@@ -1999,7 +2046,7 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
                     : launch_dec_bits<4, false>(w.attr_set, a, p.grid_x, p.lds, fz, p64, fu, x, st);
     } else if (p.route == kRoutePrefill) {
         const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y);
-        if (h->bits == 4) {
+        if (h->bits == 4 && !p.pf_i8) {
             Pf4Args pa{};
             pa.R = reinterpret_cast<const char*>(s.rec);
             pa.M = M;
@@ -2040,6 +2087,7 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
             pa.W = reinterpret_cast<const char*>(h->W);
             pa.WS = reinterpret_cast<const char*>(h->WS);
             pa.S = reinterpret_cast<const char*>(h->S);
+            pa.Z = reinterpret_cast<const char*>(h->Z);
             pa.R = reinterpret_cast<const char*>(s.rec);
             pa.C = dC;
             pa.M = M;
@@ -2049,10 +2097,12 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
             pa.ngrp = h->ngrp;
             pa.sc_shift = h->sc_shift;
             pa.ntiles = h->N / 16;
+            pa.nbg = h->nbg;
             const int scm = h->sc_blk ? 2 : (h->sc_shift == 31 ? 0 : 1);
             if (p.pf_rp == 0) e = launch_pf16_w8(pa, hp, scm, p.grid_x, st);
-            else e = hp ? launch_pf<true>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st)
-                        : launch_pf<false>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st);
+            else if (p.pf_i8) e = launch_pf<4, false>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st);
+            else e = hp ? launch_pf<8, true>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st)
+                        : launch_pf<8, false>(w.pf_attr, pa, scm, p.pf_rp, p.pf_ct, grid, st);
         }
     } else {
         const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y);
@@ -2560,7 +2610,7 @@ int i4_plan_query(int bits, int M, int K, int N, int flags, int n_cu, int32_t* o
     k.tiles = N / 16;
     const Plan p = plan_call(h, M, k, n_cu);
     const int32_t v[] = {p.route, p.quant, p.fused, p.p64, p.lrec, p.rs, p.RG, p.NG, p.pair_xcd, p.lds,
-                         p.pf_rp, p.pf_ct, p.grid_x, p.grid_y, p.split, p.stream, p.flow, p.pf_ahead, p.pf_zp};
+                         p.pf_rp, p.pf_ct, p.grid_x, p.grid_y, p.split, p.stream, p.flow, p.pf_ahead, p.pf_zp, p.pf_i8};
     const int n = std::min(nout, (int)(sizeof(v) / sizeof(v[0])));
     for (int i = 0; i < n; ++i) out[i] = v[i];
     return n;

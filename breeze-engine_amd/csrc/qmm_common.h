@@ -600,6 +600,15 @@ constexpr int kLdsMax = 160 * 1024;
 // compiler does not see these loads: every
 // wave waits for its own with an explicit vmcnt, then the workgroup barrier
 // publishes the stage.
+//
+// INT4 weights (BITS 4: explicit zero points under INT8 activations) take
+// the same core.  A stage is one INT4 chunk (four blocks, 1 KB per tile),
+// loaded raw into chunk 0's weight area; its scales and zero points go to
+// one raw area shared by both stages.  After the stage barrier all 512
+// threads expand it in place: per byte, b = nibble - zp as a signed byte
+// (n + (128 - zp)) ^ 0x80, chunk 0 getting blocks 0-1 and chunk 1 blocks 2-3
+// in the INT8 chunk layout, and the scales in that layout too.  A second
+// barrier publishes the expanded stage.
 
 constexpr int kPfWaves = 8;
 // Chunks per ring stage.
@@ -613,41 +622,60 @@ constexpr int kRecA = 2048, kRecBytes = kRecA + 128;
 // Byte of (row r, k-octet o) in a block's h half of a record.
 __host__ __device__ constexpr int pf_rec_byte(int r, int o) { return 16 * (r + 16 * (o >> 1)) + 8 * (o & 1); }
 // Byte of (column c, k-octet o) of block b in a weight tile's 1 KB in LDS.
-// Tiles arrive by DMA in the decode chunk order (octet o of both blocks at
-// 16 (c + 16 o)), so a 32x32x32 B operand takes two 8-byte halves.
-__host__ __device__ constexpr int pf_w_byte(int c, int o, int b) { return 16 * (c + 16 * o) + 8 * b; }
+// INT8 tiles arrive by DMA in the decode chunk order (octet o of both blocks
+// at 16 (c + 16 o)), so a 32x32x32 B operand takes two 8-byte halves.  INT4
+// tiles are expanded in LDS into [column half][k half][block][column c & 7]
+// [16 B]: one conflict-free 16-byte read per operand.
+__host__ __device__ constexpr int pf_w_byte(int bits, int c, int o, int b) {
+    return bits == 8 ? 16 * (c + 16 * o) + 8 * b : 16 * ((c & 7) + 8 * b + 16 * (o >> 1) + 32 * (c >> 3)) + 8 * (o & 1);
+}
 
 struct PfArgs {
-    const char* W;   // [ntiles][nch][64 lanes][16 B]
-    const char* WS;  // [ntiles][nch][16][2] int32
+    const char* W;   // INT8: [ntiles][nch][64 lanes][16 B]; INT4: [ntiles][nbg][64][16 B]
+    const char* WS;  // INT8: [ntiles][nch][16][2] int32
     const char* S;   // scales (grp_index / blk_index layouts)
+    const char* Z;   // INT4: zero points [ntiles][nbg][16][4]
     const char* R;   // activation records [Mpad/16][nch][kRecBytes]
     float* C;        // [M][N]
     int M, N, nblk, nch, ngrp, sc_shift, ntiles;
+    int nbg;         // INT4: 4-block chunks per tile
 };
 
 // SCM: scale layout: 0 one per column, 1 per group of >= 2 blocks, 2 per block.
 // One chunk's LDS region: [CT weight tiles, 1 KB each][weight sums, 128 B
-// per tile][block or group scales][2 RP activation records].
-template <int CT, int SCM, int RP, int S>
+// per tile][block or group scales][2 RP activation records].  INT4 adds kNRaw
+// raw areas after the S stages, stage g using area g % kNRaw: S - 1 when a
+// barrier follows the expansion (only the next stage waits for its expansion
+// while the one after it loads), S with one row pair, whose waves expand
+// their own tiles with no barrier after it (a wave may load stage g + S - 1
+// while another still expands stage g).  A raw area holds block scales, then
+// zero points (256 + 64 B per tile), in whole KB.
+template <int CT, int SCM, int BITS, int RP, int S>
 struct PfLayout {
     static constexpr int kWS = CT * 1024;
     static constexpr int kSB = kWS + CT * 128;
     static constexpr int kSharedUsed = kSB + (SCM == 2 ? CT * 128 : SCM == 1 ? CT * 64 : 0);
-    // The sums and scales are padded to whole KB: their 1 KB loads start
+    // INT8 pads the sums and scales to whole KB: their 1 KB loads start
     // where the weight tiles end and must not run into the records.
-    static constexpr int kShared = kWS + (kSharedUsed - kWS + 1023) / 1024 * 1024;
+    static constexpr int kShared = BITS == 8 ? kWS + (kSharedUsed - kWS + 1023) / 1024 * 1024 : kSharedUsed;
     static constexpr int kA = kShared;
     static constexpr int kChunk = kA + 2 * RP * kRecBytes;
     static constexpr int kStage = kPfChunks * kChunk;
-    // Per chunk: CT weight tiles of 1 KB, kWJ a wave; then the sums and
-    // scales in kSU units of 1 KB, kSJ a wave.
-    static constexpr int kWJ = (CT + kPfWaves - 1) / kPfWaves;
-    static constexpr int kSU = (kShared - kWS) / 1024;
+    static constexpr int kRawZ = CT * 256;  // zero points after the block scales
+    static constexpr int kRawUsed = BITS == 8 ? 0 : CT * 320;
+    static constexpr int kRaw = (kRawUsed + 1023) / 1024 * 1024;
+    static constexpr int kRawOff = S * kStage;  // raw area r at kRawOff + r * kRaw
+    static constexpr int kNRaw = RP == 1 ? S : S - 1;
+    // INT8, per chunk: CT weight tiles of 1 KB, kWJ a wave; then the sums
+    // and scales in kSU units of 1 KB, kSJ a wave.
+    static constexpr int kWJ = BITS == 8 ? (CT + kPfWaves - 1) / kPfWaves : 0;
+    static constexpr int kSU = BITS == 8 ? (kShared - kWS) / 1024 : 0;
     static constexpr int kSJ = (kSU + kPfWaves - 1) / kPfWaves;
-    // Shared loads a wave issues per chunk.
-    static constexpr int kPerWave = kWJ + kSJ;
-    static constexpr int kBytes = S * kStage;
+    // INT4, per stage: the CT raw tiles and the raw area in units of 1 KB.
+    static constexpr int kUnits = CT + kRaw / 1024;
+    // Shared loads a wave issues per chunk (INT8) or stage (INT4).
+    static constexpr int kPerWave = BITS == 8 ? kWJ + kSJ : (kUnits + kPfWaves - 1) / kPfWaves;
+    static constexpr int kBytes = kRawOff + kNRaw * kRaw;
     static_assert(kShared % 64 == 0 && kBytes <= 160 * 1024, "layout");
 };
 
@@ -919,7 +947,7 @@ hipError_t launch_dec_bits(bool* attr_set, const GemvArgs& a, int grid, int lds,
 template <int BITS, bool HP>
 hipError_t launch_dec8(bool* attr_set, const GemvArgs& a, const uint4* rec, int grid, int lds, int fuse, bool extra,
                        bool lrec, hipStream_t st);
-template <bool HP>
+template <int BITS, bool HP>
 hipError_t launch_pf(bool* pf_attr, const PfArgs& p, int scm, int rp, int ct, dim3 grid, hipStream_t st);
 hipError_t launch_pf16(const Pf4Args& p, bool zp, int ahead, int grid, hipStream_t st);
 hipError_t launch_pf16_w8(const PfArgs& p, bool hp, int scm, int grid, hipStream_t st);

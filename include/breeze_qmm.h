@@ -158,7 +158,7 @@ int i4_rmsnorm_matmul_multi_dev(const float* dX, const float* dNormW, float eps,
  * handle.  flags: 1 block-integer export, 2 argmax, 4 gate/up pair,
  * 8 multi-projection (one segment of N), 16 RMSNorm in that launch,
  * 32 per-block metadata (small scale groups), 64 legacy corr, 128 explicit
- * zero points, 256 INT8 activations; n_cu: compute units of the device.  out[0..18] = route
+ * zero points, 256 INT8 activations; n_cu: compute units of the device.  out[0..19] = route
  * (1 decode in four-row groups, 2 decode in eight-row groups, 3 prefill
  * GEMM, 4 rows kernel, 0 no single launch takes a paired or multi call),
  * stand-alone quantizer (0 none: the decode prologue quantizes, 1 staged
@@ -168,8 +168,8 @@ int i4_rmsnorm_matmul_multi_dev(const float* dX, const float* dNormW, float eps,
  * (0: independent 16-row waves), prefill column tiles, grid x, grid y,
  * split-K workgroups per tile (0: none), non-temporal weight loads, phases
  * across tile boundaries, weight chunks in flight of the independent waves
- * (INT4), INT4 prefill with zero points.  Environment overrides apply as for
- * a call.  Returns the number of values written (at most nout), or -1. */
+ * (INT4), INT4 prefill with zero points, INT4 prefill on the INT8 matrix
+ * instructions.  Environment overrides apply as for a call.  Returns the number of values written (at most nout), or -1. */
 int i4_plan_query(int bits, int M, int K, int N, int flags, int n_cu, int32_t* out, int nout);
 
 /* Handle facts: out[0..7] = N, K, bits, scale group (blocks per distinct

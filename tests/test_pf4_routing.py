@@ -128,3 +128,23 @@ def test_every_output_is_covered_in_every_mode(hb, M, N, call):
         assert p["grid_x"] * 4 >= tiles * -(-M // 16)
     else:
         assert p["grid_x"] * p["pf_ct"] >= tiles and p["grid_y"] * 32 * p["pf_rp"] >= M
+
+
+def test_zero_points_under_int8_activations(hb, monkeypatch):
+    """One projection past 64 rows with explicit zero points, INT8 activations:
+    the INT8 instructions where their cost is less."""
+    call = dict(zeros=True, hi=False)
+    assert hb.plan(4, 128, 5120, 17408, **call)["pf_i8"] == 1
+    assert hb.plan(4, 400, 1024, 5120, **call)["pf_i8"] == 1
+    assert hb.plan(4, 1024, 2048, 17408, **call)["pf_i8"] == 1
+    assert hb.plan(4, 320, 5120, 2560, **call)["pf_i8"] == 0    # FP6, (2, 4)
+    assert hb.plan(4, 96, 5120, 5120, **call)["pf_rp"] == 0     # independent waves
+    assert hb.plan(4, 64, 5120, 17408, **call)["pf_i8"] == 0
+    assert hb.plan(4, 128, 5120, 17408, pair=True, **call)["pf_i8"] == 0
+    assert hb.plan(4, 128, 5120, 17408, hi=False, extra=True)["pf_i8"] == 0
+    assert hb.plan(4, 128, 5120, 17408, zeros=True)["pf_i8"] == 0
+    assert hb.plan(8, 128, 5120, 17408, hi=False)["pf_i8"] == 0
+    monkeypatch.setenv("BREEZE_HIP_PF_I8", "0")
+    assert hb.plan(4, 128, 5120, 17408, **call)["pf_i8"] == 0
+    monkeypatch.setenv("BREEZE_HIP_PF_I8", "1")
+    assert hb.plan(4, 64, 5120, 17408, **call)["pf_i8"] == 1

@@ -434,9 +434,10 @@ int pick_pf_rp(int M, const char* force) {
 // Column tiles per workgroup for rp row pairs: among the instantiated
 // widths, the one that minimizes (workgroup rounds at one workgroup per CU)
 // x (tiles on the busiest SIMD, whose two waves hold column parts s / rp and
-// (s + 4) / rp); *rounds receives the rounds.  `force` (BREEZE_HIP_PREFILL_CT)
-// selects an instantiated width for rp instead, for tests and tuning.
-int pick_pf_ct(int ntiles, int gy, int rp, int n_cu, const char* force, int* rounds) {
+// (s + 4) / rp), which *rounds and *simd_tiles receive.  `force`
+// (BREEZE_HIP_PREFILL_CT) selects an instantiated width for rp instead, for
+// tests and tuning.
+int pick_pf_ct(int ntiles, int gy, int rp, int n_cu, const char* force, int* rounds, int* simd_tiles) {
     if (force) {
         const int v = std::atoi(force);
         for (const PfCfg& c : kPfCfgs)
@@ -458,6 +459,7 @@ int pick_pf_ct(int ntiles, int gy, int rp, int n_cu, const char* force, int* rou
             best_cost = cost;
             best = c.ct;
             *rounds = (int)((wgs + n_cu - 1) / n_cu);
+            *simd_tiles = simd;
         }
     }
     return best;
@@ -1221,11 +1223,17 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //     and the block-integer export).
 //   pick_pf_rp  32-row prefill workgroups up to 32 rows, 64 up to 64, then
 //     128 (the C4 shape's 512 rows fill the CUs with 128-row workgroups).
-//   kPf16TilesPerCu8 (13)  the same for INT8 (pf16_w8_kernel).  Workgroups
-//     (prefill_kernel) against independent waves, K=5120: N=5120 at 33 / 64 /
-//     128 / 200 rows (4 / 5 / 10 / 16 tiles a CU) 47 / 47 / 58 / 60 -> 21 / 32 /
-//     44 / 70; N=17408 at 32 / 48 / 64 rows (9 / 13 / 17) 46 / 63 / 63 -> 45 /
-//     57 / 67; K=17408 N=5120 at 48 rows 145 -> 59.
+//   kPf16Cost8, pf8_cost  an INT8 prefill of up to 13 output tiles of 16x16 a
+//     CU (kPf16TilesPerCu) runs as independent 16-row waves (pf16_w8_kernel)
+//     where these cost less than workgroups (prefill_kernel).  A wave's time
+//     steps with the workgroups on the busiest CU, by 70 ns a block in two
+//     passes, 85 with per-block scales, 49 and 60 with INT8 activations;
+//     workgroups hardly depend on the scales.  Workgroups -> waves, K=5120:
+//     N=5120 at 33 / 64 / 128 rows 47 / 47 / 58 -> 21 / 31 / 43; kept on
+//     workgroups with per-block scales: N=17408 at 48 rows 56 (waves 64),
+//     N=10240 at 80 rows 55 (65), K=12288 N=17408 at 24 / 33 rows 104 / 127
+//     (135 / 171), K=1024 N=17408 at 33 rows 16.2 (19.2).  Past 13 tiles a CU
+//     N=5120 at 200 rows takes 60 on workgroups, 70 on waves.
 //   kPf16TilesPerCu (13), kPf16DeepPerCu (6)  the INT4 prefill runs as
 //     independent 16-row waves (pf16_kernel) up to 13 output tiles of 16x16 a
 //     CU, with four weight chunks in flight up to 6 tiles a CU and two past
@@ -1328,7 +1336,7 @@ constexpr int kPairMaxRows4 = 16;
 constexpr int kDec8LrecTiles = 2;
 constexpr int kPrefillMinRows = 9;
 constexpr int kSplitMaxTiles = 8, kSplitMinPhases = 20;
-constexpr int kPf16TilesPerCu = 13, kPf16TilesPerCu8 = 13, kPf16DeepPerCu = 6;
+constexpr int kPf16TilesPerCu = 13, kPf16DeepPerCu = 6;
 constexpr int kStreamIdleDiv = 8, kStreamMaxGroups = 2;
 
 // Row-blocks the decode prologue quantizes itself for calls of M rows
@@ -1518,7 +1526,7 @@ int split_pieces(const Shape& h, int M, const CallKind& k, int n_cu, int* lds) {
     return S;
 }
 
-// What an INT4 prefill call takes by its launch, in ns (see the routing table).
+// What a prefill call takes by its launch, in ns (see the routing table).
 //
 // Independent 16-row waves: per workgroup of the busiest CU `start` ns and
 // `per` ns a block, besides `once` ns a block.
@@ -1529,9 +1537,17 @@ double pf16_cost(const Pf16Cost& c, int nblk, long waves, int n_cu) {
     const long wgs = (waves + kPf16Waves - 1) / kPf16Waves, n = (wgs + n_cu - 1) / n_cu;
     return 4550.0 + (double)(n * c.start) + nblk * (c.once + (double)(n * c.per));
 }
-// By (explicit zero points, four weight chunks in flight).
+// INT8 weights, by (two-pass, per-block scales).
+constexpr Pf16Cost kPf16Cost8[2][2] = {{{550, 5, 49}, {550, 10, 60}}, {{700, 24, 70}, {700, 20, 85}}};
+// Their workgroups (prefill_kernel): rounds of one a CU, `simd` tiles on the
+// busiest SIMD; a block takes a tenth less where one of four row pairs idles.
+double pf8_cost(int nblk, int rounds, int simd, bool hp, bool idle) {
+    const double ns = (hp ? 160 + 44 * simd : 155 + 28 * simd) * (idle ? 0.9 : 1.0);
+    return 4900.0 + (double)rounds * (400 * simd + nblk * ns);
+}
+// INT4, by (explicit zero points, four weight chunks in flight).
 constexpr Pf16Cost kPf16Cost4[2][2] = {{{550, 97, 57}, {550, 76, 47}}, {{800, 66, 80}, {800, 58, 74}}};
-// Workgroup shapes: ns a block of one round, for two-pass calls, two-pass with
+// INT4 workgroup shapes: ns a block of one round, for two-pass calls, two-pass with
 // zero points, INT8 activations, and those with zero points.  Shapes of four
 // waves run two workgroups a CU; `half` is for a single round of one.  `i8`:
 // the same shape on the INT8 matrix instructions (pf4_i8).
@@ -1609,18 +1625,19 @@ bool take_pf4_i8(const Shape& h, const CallKind& k, int M, double cost, double f
 }
 
 // Whether a prefill call of few output tiles a CU runs as independent 16-row
-// waves, given what INT4 workgroups would take (see the routing table).
+// waves, given what its workgroups would take (see the routing table).
 // BREEZE_HIP_PF16=0 / 1 turns them off / on; a forced workgroup shape turns
 // them off.
 bool pick_pf16(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, int n_cu, double wg_cost) {
     const char* env = std::getenv("BREEZE_HIP_PF16");
     const long waves = (long)tiles * ((M + 15) / 16);
     const bool deep = waves <= (long)kPf16DeepPerCu * n_cu;
-    const long most = (long)(h.bits == 4 ? kPf16TilesPerCu : kPf16TilesPerCu8) * n_cu;
-    bool take = waves <= most && !std::getenv("BREEZE_HIP_PREFILL_RP") &&
+    bool take = waves <= (long)kPf16TilesPerCu * n_cu && !std::getenv("BREEZE_HIP_PREFILL_RP") &&
                 !std::getenv("BREEZE_HIP_PREFILL_CT");
-    if (take && h.bits == 4 && !pf4_plain(h, k))
-        take = pf16_cost(kPf16Cost4[h.has_zp][deep], h.nblk, waves, n_cu) <= wg_cost;
+    if (take && !(h.bits == 4 && pf4_plain(h, k))) {
+        const Pf16Cost& c = h.bits == 8 ? kPf16Cost8[k.hp][h.extra] : kPf16Cost4[h.has_zp][deep];
+        take = pf16_cost(c, h.nblk, waves, n_cu) <= wg_cost;
+    }
     if (!(env ? env[0] == '1' : take)) return false;
     p.pf_rp = 0;
     p.pf_ct = 1;
@@ -1705,8 +1722,8 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
         const int rows = 32 * p.pf_rp;
         p.Mpad = (M + rows - 1) / rows * rows;
         p.grid_y = p.Mpad / rows;
-        int rounds = 1;
-        const int ct = pick_pf_ct(tiles, p.grid_y, p.pf_rp, n_cu, std::getenv("BREEZE_HIP_PREFILL_CT"), &rounds);
+        int rounds = 1, simd = 1;
+        const int ct = pick_pf_ct(tiles, p.grid_y, p.pf_rp, n_cu, std::getenv("BREEZE_HIP_PREFILL_CT"), &rounds, &simd);
         if (h.bits == 4) {
             Plan i8 = p;
             i8.pf_i8 = true;
@@ -1721,7 +1738,8 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
             pick_pf16(p, h, k, M, tiles, n_cu, cost);
             return p;
         }
-        if (pick_pf16(p, h, k, M, tiles, n_cu, 0.0)) return p;
+        const bool idle = p.grid_y == 1 && p.pf_rp == 4 && M <= 96;
+        if (pick_pf16(p, h, k, M, tiles, n_cu, pf8_cost(h.nblk, rounds, simd, k.hp, idle))) return p;
         p.pf_ct = ct;
         p.grid_x = (tiles + p.pf_ct - 1) / p.pf_ct;
     } else if (dec8) {

@@ -634,11 +634,12 @@ struct PfArgs {
     const char* W;   // INT8: [ntiles][nch][64 lanes][16 B]; INT4: [ntiles][nbg][64][16 B]
     const char* WS;  // INT8: [ntiles][nch][16][2] int32
     const char* S;   // scales (grp_index / blk_index layouts)
-    const char* Z;   // INT4: zero points [ntiles][nbg][16][4]
     const char* R;   // activation records [Mpad/16][nch][kRecBytes]
     float* C;        // [M][N]
     int M, N, nblk, nch, ngrp, sc_shift, ntiles;
-    int nbg;         // INT4: 4-block chunks per tile
+    // INT4: 4-block chunks per tile, zero points [ntiles][nbg][16][4].
+    int nbg;
+    const char* Z;
 };
 
 // SCM: scale layout: 0 one per column, 1 per group of >= 2 blocks, 2 per block.

@@ -148,3 +148,21 @@ def test_zero_points_under_int8_activations(hb, monkeypatch):
     assert hb.plan(4, 128, 5120, 17408, **call)["pf_i8"] == 0
     monkeypatch.setenv("BREEZE_HIP_PF_I8", "1")
     assert hb.plan(4, 64, 5120, 17408, **call)["pf_i8"] == 1
+
+
+@pytest.mark.parametrize("shape,call,waves", [
+    ((64, 5120, 5120), dict(), True),
+    ((64, 5120, 5120), dict(extra=True), True),
+    ((64, 5120, 5120), dict(hi=False, extra=True), True),
+    ((128, 5120, 5120), dict(), True),
+    ((48, 5120, 17408), dict(extra=True), False),   # four workgroups on the busiest CU
+    ((48, 5120, 17408), dict(hi=False), True),
+    ((80, 5120, 10240), dict(extra=True), False),
+    ((24, 12288, 17408), dict(extra=True), False),
+    ((33, 1024, 17408), dict(extra=True), False),
+    ((320, 5120, 2560), dict(extra=True), False),
+])
+def test_int8_waves_where_they_cost_less(hb, shape, call, waves):
+    """Per-block scales make the independent waves' step longer, INT8
+    activations shorter; workgroups change little."""
+    assert (hb.plan(8, *shape, n_cu=256, **call)["pf_rp"] == 0) == waves

@@ -916,10 +916,16 @@ Scratch* scratch_for(Workspace& w, hipStream_t st) {
 // share the array and race.
 constexpr size_t kNoAllocBytes = 16u << 20;
 constexpr size_t kNoAllocState = 512;
-// A call's room is counted in the INT8 GEMM's record bytes, so what fits does
-// not depend on the weights' width; the FP6 records of the INT4 GEMM take
-// 4096 / 2176 of that.
-constexpr size_t kNoAllocArray = (kNoAllocBytes / kRecBytes + 1) * 2 * kF6Rec;
+// A call's room is counted in prefill_kernel's record bytes, kRecBytes per
+// (16 rows, two blocks), so what fits depends neither on the weights' width
+// nor on the launch; the array holds as many of the largest records: FP6 ones
+// take 4,096 bytes there (kRecMost), the independent INT8 waves' up to 2,560.
+constexpr size_t kRecMost = 2 * kF6Rec;
+static_assert(kRecBytes <= kRecMost && (size_t)r16_rec_bytes(true) <= kRecMost, "the largest prefill record");
+constexpr size_t kNoAllocArray = (kNoAllocBytes / kRecBytes + 1) * kRecMost;
+// State and records without partials; a byte of partials takes 1.9 of records.
+static_assert(kNoAllocState + (kNoAllocBytes - kNoAllocState) / kRecBytes * kRecMost <= kNoAllocArray / 256 * 256,
+              "the records of an accepted call fit");
 static __device__ __align__(256) uint8_t scratch[kNoAllocArray];
 uint8_t* g_noalloc_ptr[kMaxDevices];
 
@@ -1878,30 +1884,29 @@ int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, 
 
     // The stand-alone quantizer ahead of the matmul kernel.
     if (p.quant == kQuantPrefill) {
-        // Records in MFMA operand order for the prefill GEMM.
+        // Records in MFMA operand order for the prefill GEMM.  The stream's
+        // room for them is counted for the largest kind, so it depends on the
+        // rows and K alone: a call of no more rows than an earlier one needs
+        // no allocation, whatever its launch and weights (a capturing stream
+        // could not make one).  The fixed scratch counts kRecBytes.
         const int nch_rec = (h->nblk + 1) / 2;  // record chunks of two blocks
-        const size_t int8_bytes = (size_t)(p.Mpad / 16) * nch_rec * kRecBytes;
+        const size_t chunks = (size_t)(p.Mpad / 16) * nch_rec;
+        if (!grow(w, st, &s.rec, &s.rec_cap, chunks * (s.fixed ? kRecBytes : kRecMost), "workspace alloc", s.fixed))
+            return -4;
         if (h->bits == 4 && !p.pf_i8) {
             const int rtiles = (M + 31) / 32 * 2, mult = p.pf_zp ? 1 : 8;
-            // The fixed scratch counts the INT8 records' bytes (the array is
-            // larger by the FP6 records' share, kNoAllocArray).
-            const size_t bytes = s.fixed ? int8_bytes : (size_t)rtiles * h->nblk * kF6Rec;
-            if (!grow(w, st, &s.rec, &s.rec_cap, bytes, "workspace alloc", s.fixed)) return -4;
             const size_t waves = (size_t)rtiles * h->nblk;  // a wave per (16 rows, block)
             const unsigned qb = (unsigned)((waves + 3) / 4);
             if (hp) quantize_f6_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, rtiles, mult, s.rec);
             else quantize_f6_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, rtiles, mult, s.rec);
         } else if (p.pf_rp == 0) {  // INT8 weights
             const int rtiles = (M + 15) / 16;
-            const size_t bytes = s.fixed ? int8_bytes : (size_t)rtiles * nch_rec * r16_rec_bytes(hp);
-            if (!grow(w, st, &s.rec, &s.rec_cap, bytes, "workspace alloc", s.fixed)) return -4;
             const size_t waves = (size_t)rtiles * h->nblk;
             const unsigned qb = (unsigned)((waves + 3) / 4);
             if (hp) quantize_r16_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, rtiles, s.rec);
             else quantize_r16_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, rtiles, s.rec);
         } else {
-            if (!grow(w, st, &s.rec, &s.rec_cap, int8_bytes, "workspace alloc", s.fixed)) return -4;
-            const size_t threads = (size_t)(p.Mpad / 16) * nch_rec * 2 * 64;  // a wave per (16 rows, block)
+            const size_t threads = chunks * 2 * 64;  // a wave per (16 rows, block)
             const unsigned qb = (unsigned)((threads + 255) / 256);
             if (hp) quantize_rec_kernel<true><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, p.Mpad, s.rec);
             else quantize_rec_kernel<false><<<qb, 256, 0, st>>>(dA, M, h->K, h->nblk, nch_rec, p.Mpad, s.rec);

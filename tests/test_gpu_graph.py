@@ -86,3 +86,50 @@ def test_captured_argmax_replays_exact(gpu, hb, hi_prec):
             torch.cuda.synchronize()
     finally:
         hb.free(h)
+
+
+@pytest.mark.parametrize("first,then", [
+    ((8, 256), (8, 240)),   # workgroups, then independent waves (larger records a row)
+    ((8, 128), (4, 128)),   # INT8 weights, then INT4 (FP6 records)
+    ((4, 128), (8, 128)),
+])
+def test_capture_after_a_call_of_as_many_rows(gpu, hb, orc, hi_prec, first, then):
+    """A stream's room for the prefill's records depends on the rows and K
+    alone, so after one call a call of no more rows is captured without an
+    allocation, whatever its launch and weights; replays are bit-exact with
+    eager work between them."""
+    torch = gpu
+    K, N = 1024, 3536
+    rng = np.random.default_rng(first[1])
+    handles, weights = {}, {}
+    for bits in (4, 8):
+        qw, sc, _ = rng_weights(rng, N, K, bits)
+        sc = np.ascontiguousarray(np.repeat(sc[:, :1], K // 32, axis=1))
+        weights[bits] = (qw, sc)
+        handles[bits] = hb.prepack(qw, sc, None, K, N, bits=bits)
+    hb.set_hi_prec(True)
+    if first[0] == then[0] == 8:
+        assert hb.plan(8, first[1], K, N)["pf_rp"] == 4 and hb.plan(8, then[1], K, N)["pf_rp"] == 0
+    try:
+        cap = torch.cuda.Stream()
+        a0 = torch.from_numpy(rng.normal(size=(first[1], K)).astype(np.float32)).cuda()
+        A = [rng.normal(size=(then[1], K)).astype(np.float32) for _ in range(3)]
+        x = torch.from_numpy(A[0]).cuda()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(cap):
+            hb.matmul(handles[first[0]], a0, N)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=cap):
+            y = hb.matmul(handles[then[0]], x, N)
+        for a in A:
+            x.copy_(torch.from_numpy(a))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert bits_equal(y.cpu().numpy(), orc.matmul(*weights[then[0]], None, N, K, then[0], a, True))
+            with torch.cuda.stream(cap):
+                hb.matmul(handles[first[0]], a0, N)
+            torch.cuda.synchronize()
+    finally:
+        for h in handles.values():
+            hb.free(h)

@@ -1329,7 +1329,8 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 // every prologue-quantized call), BREEZE_HIP_DEC8_ROWS (their row limit),
 // BREEZE_HIP_DEC8_LREC (0: records never in LDS; n: from n tiles),
 // BREEZE_HIP_PREFILL_RP / _CT (prefill workgroup shape), BREEZE_HIP_PF16 (the
-// prefill's independent waves: 0 never, 1 always), BREEZE_HIP_PF_I8 (INT4
+// prefill's independent waves: 0 never, 1 always) and BREEZE_HIP_PF16_AHEAD
+// (their weight chunks in flight, INT4), BREEZE_HIP_PF_I8 (INT4
 // prefill on the INT8 instructions: 0 never, 1 where it can), BREEZE_HIP_FUSED_MAX_BLOCKS
 // (row-blocks the decode prologue quantizes), BREEZE_HIP_SPLIT (split-K),
 // BREEZE_HIP_STREAM (non-temporal weight loads), BREEZE_HIP_FLOW (phases
@@ -1632,8 +1633,8 @@ bool take_pf4_i8(const Shape& h, const CallKind& k, int M, double cost, double f
 
 // Whether a prefill call of few output tiles a CU runs as independent 16-row
 // waves, given what its workgroups would take (see the routing table).
-// BREEZE_HIP_PF16=0 / 1 turns them off / on; a forced workgroup shape turns
-// them off.
+// BREEZE_HIP_PF16=0 / 1 turns them off / on (a forced workgroup shape turns
+// them off), BREEZE_HIP_PF16_AHEAD=2 / 4 sets INT4's chunks in flight.
 bool pick_pf16(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, int n_cu, double wg_cost) {
     const char* env = std::getenv("BREEZE_HIP_PF16");
     const long waves = (long)tiles * ((M + 15) / 16);
@@ -1649,6 +1650,7 @@ bool pick_pf16(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, int
     p.pf_ct = 1;
     p.pf_i8 = false;
     p.pf_ahead = deep ? 4 : 2;
+    if (const char* ahead = std::getenv("BREEZE_HIP_PF16_AHEAD")) p.pf_ahead = ahead[0] == '2' ? 2 : 4;
     p.grid_x = (int)((waves + kPf16Waves - 1) / kPf16Waves);
     p.grid_y = 1;
     return true;

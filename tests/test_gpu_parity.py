@@ -184,9 +184,8 @@ def test_legacy_int4_signed_zero_points(gpu, hb, orc, hi_prec, zp_lo, zp_hi):
     """Legacy INT4 handles keep signed int8 zero points from -112 up
     (b = nibble - zp never wraps there) with a consistent corr, so they stay
     INT4 with explicit zero points: the decode kernel (1, 3, 8, 9, 17 rows)
-    and the prefill GEMM's in-LDS nibble expansion (33, 130 rows), whose per-byte
-    n - zp must not borrow across bytes for negative zp.  33 blocks: a
-    partial last 4-block chunk."""
+    and the prefill (33, 130 rows), where the zero point is a factor of the
+    row sums.  33 blocks: a partial last 4-block chunk."""
     N, K = 64, 1056
     nblk = K // 32
     rng = np.random.default_rng(zp_lo + 1000)
@@ -363,8 +362,8 @@ def test_prefill_gemm_bit_exact(gpu, hb, orc, hi_prec, monkeypatch, scales, cfg)
 @pytest.mark.parametrize("scales", ["channel", "group4", "group8", "block", "zeros"])
 @pytest.mark.parametrize("cfg", PF_CFGS)
 def test_prefill_gemm_int4_bit_exact(gpu, hb, orc, hi_prec, monkeypatch, scales, cfg):
-    """The M > 8 GEMM on INT4 weights (nibbles expanded to signed bytes
-    n - zp in LDS) against the oracle: per-column scales, groups of one and
+    """The M > 8 GEMM on INT4 weights (FP6 matrix instructions; every shape of
+    kPfCfgs, (4, 5) too, is the one that runs) against the oracle: per-column scales, groups of one and
     two 4-block chunks, per-block scales (default zero point 8) and explicit
     zero points 0..15; every workgroup shape with a partial last column
     group (19 tiles); 33 and 35 blocks, so the last 4-block chunk holds one

@@ -166,3 +166,22 @@ def test_int8_waves_where_they_cost_less(hb, shape, call, waves):
     """Per-block scales make the independent waves' step longer, INT8
     activations shorter; workgroups change little."""
     assert (hb.plan(8, *shape, n_cu=256, **call)["pf_rp"] == 0) == waves
+
+
+def test_weight_chunks_in_flight(hb, monkeypatch):
+    """Four up to six output tiles a CU, two past that."""
+    assert hb.plan(4, 33, 5120, 5120)["pf_ahead"] == 4               # 960 waves
+    assert hb.plan(4, 77, 5120, 5120, zeros=True, hi=False)["pf_ahead"] == 2  # 1600
+    assert hb.plan(4, 166, 4096, 4096)["pf_ahead"] == 2              # 2816
+    monkeypatch.setenv("BREEZE_HIP_PF16_AHEAD", "2")
+    assert hb.plan(4, 33, 5120, 5120)["pf_ahead"] == 2
+
+
+@pytest.mark.parametrize("zeros", [False, True])
+def test_every_shape_can_be_forced(hb, monkeypatch, zeros):
+    for rp, cts in ((4, (17, 16, 13, 12, 9, 8, 5, 4)), (2, (16, 8, 4)), (1, (16, 8))):
+        monkeypatch.setenv("BREEZE_HIP_PREFILL_RP", str(rp))
+        for ct in cts:
+            monkeypatch.setenv("BREEZE_HIP_PREFILL_CT", str(ct))
+            p = hb.plan(4, 130, 1056, 304, zeros=zeros)
+            assert (p["pf_rp"], p["pf_ct"]) == (rp, ct)

@@ -4,7 +4,7 @@ routing change shows here and not only as time.  CPU only: the plan is made
 from the shape alone.
 
 Routes: "decode" (dec_kernel, row groups of up to four), "decode8"
-(dec8_kernel, row groups of eight), "prefill" (the INT8-MFMA GEMM), "rows"
+(dec8_kernel, row groups of eight), "prefill" (the GEMMs past them), "rows"
 (the rows kernel: block-integer export, legacy corr past the decode rows),
 None (no single launch takes a paired or multi-projection call; the library
 then runs the projections one by one).  Quantizer: None when the decode

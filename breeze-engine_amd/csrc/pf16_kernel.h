@@ -16,7 +16,7 @@ namespace bq {
 //
 // No barriers: a wave expands its own weights in its own LDS.  AHEAD chunks
 // of weights are in flight in registers: four while the waves are few, two
-// past that (113 registers: four waves a SIMD).
+// past that (107 registers, 110 with zero points: four waves a SIMD).
 constexpr int kPf16Stage = 2048;  // LDS of one stage (four blocks) of a wave: 64 operands of 32 B
 
 template <bool ZP, int AHEAD>

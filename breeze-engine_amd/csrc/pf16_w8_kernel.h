@@ -9,7 +9,7 @@ namespace bq {
 // Bound: one wave's chain per block (two matrix instructions, sixteen
 // dependent vector instructions) and the CU's vector memory issue.  Weights
 // are the matrix operand as they lie in memory and records are written in
-// operand order (kR16Rec), so a block is three 1 KB loads a wave (its half of
+// operand order (r16_rec_bytes), so a block is three 1 KB loads a wave (its half of
 // the weight chunk and of its sums and scales among them) and there is no LDS
 // and no barrier.  The workgroups of prefill_kernel (32 RP rows) leave most
 // CUs without one here.

@@ -1448,7 +1448,7 @@ struct CallKind {
 };
 
 struct Plan {
-    int route = kRouteNone;  // kRouteNone: a paired or multi call no decode launch takes
+    int route = kRouteNone;  // kRouteNone: a paired or multi call that no one launch takes
     int quant = kQuantNone;
     bool fused = false;      // the decode prologue quantizes
     bool p64 = false;        // decode, one or two rows: block pairs on 16x16x64
@@ -1792,10 +1792,10 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
 
 // Quantize + block dots + epilogue for M rows on `st`.  Exactly one of
 // dC / dCs is non-null; dIdx (optional) receives the per-row argmax.
-constexpr int kNotPairable = -100;  // run() with h2: the decode kernel does not take this call
+constexpr int kNotPairable = -100;  // run() with h2 or mp: no one launch takes this call
 
-// Handles one decode launch can stream together: the same device and
-// device layout; the gate/up pairing also needs the same N.
+// Handles one launch can read together: the same device and device layout;
+// the gate/up pairing also needs the same N.
 bool same_layout_but_n(const Handle* a, const Handle* b) {
     return a->device == b->device && a->K == b->K && a->bits == b->bits && a->nbg == b->nbg &&
            a->sc_shift == b->sc_shift && a->ngrp == b->ngrp && a->sc_blk == b->sc_blk && a->extra == b->extra &&
@@ -1803,7 +1803,7 @@ bool same_layout_but_n(const Handle* a, const Handle* b) {
 }
 bool same_layout(const Handle* a, const Handle* b) { return a->N == b->N && same_layout_but_n(a, b); }
 
-// Projections of one activation in one decode launch (i4_matmul_multi_dev).
+// Projections of one activation in one launch (i4_matmul_multi_dev).
 struct Multi {
     const Handle* h[kMaxSeg];
     float* C[kMaxSeg];
@@ -1817,11 +1817,12 @@ struct Multi {
 };
 
 // h2 (gate/up pairing): a second handle with the same layout (same_layout).
-// Returns kNotPairable, having launched nothing, when the decode kernel does
-// not take the call.
+// Returns kNotPairable, having launched nothing, when neither a decode launch
+// nor, past 32 rows, one INT4 prefill launch takes both.
 // The caller holds w.mu; s is the scratch of st.
 // mp (multi-projection): h is mp->h[0] and dC is mp->C[0]; returns
-// kNotPairable, having launched nothing, unless one decode launch takes all.
+// kNotPairable, having launched nothing, unless one decode or INT4 prefill
+// launch takes all.
 int run(Workspace& w, Scratch& s, Handle* h, const float* dA, int M, float* dC, int32_t* dCs, int64_t* dIdx,
         hipStream_t st, const Handle* h2 = nullptr, const Multi* mp = nullptr) {
     if (M < 0) {

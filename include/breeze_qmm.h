@@ -113,14 +113,16 @@ int i4_silu_mul_dev(const float* dG, const float* dU, size_t n, float* dOut, voi
  * allocates nothing: no hipMalloc, hipFree or allocating library call.  It
  * has no counterpart in the reference; it is for callers that cannot
  * allocate, such as code under HIP graph capture or serving loops that
- * forbid it.  All of its device scratch is one static 16 MiB array per
- * device, so a call whose activation records do not fit is refused (-4,
- * i4_last_error() says why): 72 bytes per row and 32-block of K when
+ * forbid it.  All of its device scratch is one static array per device (30.1
+ * MiB of device memory while the library is loaded), of which calls are given
+ * 16 MiB by the count below, so a call whose activation records do not fit is
+ * refused (-4, i4_last_error() says why): 72 bytes per row and 32-block of K when
  * the decode kernel stages its records (up to 32 rows, M*K above 16384), with
  * K counted rounded up to a multiple of 128 and, from 5 to 32 rows, M rounded
  * up to a multiple of 8 (the eight-row groups' records cover whole groups), and
  * about 68 bytes per 32-block of K per row, rows rounded up to 32, 64 or 128, for
- * the rows the prefill GEMM takes; a split-K call (few column tiles over a long
+ * the rows the prefill GEMM takes (whatever its kernel: the array holds as
+ * many of the largest records, 128 bytes); a split-K call (few column tiles over a long
  * K) takes 4 bytes per 16-column tile rounded up to 256, plus 68 bytes per row
  * and 32-block of K (K rounded up to a multiple of 128) per tile.  Calls that
  * overlap on one device share the array and race: serialize them.  Outputs are those of i4_matmul_dev /

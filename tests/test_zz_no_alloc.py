@@ -107,7 +107,7 @@ def test_noalloc_legacy_corr_rows_kernel(gpu, hb, orc, hi_prec, bits):
 
 def test_noalloc_refuses_what_does_not_fit(gpu, hb, hi_prec):
     """Prefill records of 2048 rows x K = 17408 (about 150 MB) exceed the
-    16 MiB scratch: the call returns an error and launches nothing; the next
+    16 MiB that calls are given: the call returns an error and launches nothing; the next
     call that fits works."""
     torch = gpu
     N, K = 32, 17408
@@ -129,6 +129,38 @@ def test_noalloc_refuses_what_does_not_fit(gpu, hb, hi_prec):
         assert bits_equal(got, want)
     finally:
         hb.free(h)
+
+
+@pytest.mark.parametrize("bits,rows,hp", [(4, 130, True), (4, 130, False), (8, 130, True), (8, 48, True)])
+def test_noalloc_largest_records(gpu, hb, hi_prec, bits, rows, hp):
+    """The most blocks of K whose records the fixed scratch accepts (room is
+    counted as 2,176 bytes a 16 rows and two blocks; FP6 records take 4,096,
+    independent INT8 waves' 2,560), and four blocks more, refused alike."""
+    torch = gpu
+    N = 16
+    pad = 256 if rows > 128 else 64
+    nblk = 2 * (((16 << 20) - 512) // 2176 // (pad // 16))
+    rng = np.random.default_rng(nblk)
+    for blocks, fits in ((nblk, True), (nblk + 4, False)):
+        K = 32 * blocks
+        qw, sc, _ = rng_weights(rng, N, K, bits)
+        sc = np.ascontiguousarray(np.repeat(sc[:, :1], blocks, axis=1))
+        h = hb.prepack(qw, sc, None, K, N, bits=bits)
+        hb.set_hi_prec(hp)
+        try:
+            A = rng.normal(size=(rows, K)).astype(np.float32)
+            if fits:
+                got, _ = _noalloc(hb, torch, h, A, N, False)
+                want, _ = _reference_call(hb, torch, h, A, N, False)
+                assert bits_equal(got, want)
+            else:
+                dA, out = torch.from_numpy(A).cuda(), torch.zeros((rows, N), device="cuda")
+                st = hb._vp(torch.cuda.current_stream().cuda_stream)
+                rc = hb._lib.i4_matmul_noalloc_dev(hb._vp(h), hb._vp(dA.data_ptr()), rows, hb._vp(out.data_ptr()),
+                                                   None, st)
+                assert rc == -4, rc
+        finally:
+            hb.free(h)
 
 
 def test_noalloc_inside_graph_capture(gpu, hb, hi_prec):

@@ -11,7 +11,7 @@ namespace bq {
 // CU's vector memory issue (16 cycles per 1 KB load: a record is two, a chunk
 // of weights one per four blocks).  A tile of 32 rows by 32 columns a wave
 // (pf4_kernel) needs a quarter of the loads but leaves most SIMDs without a
-// wave: K=5120 N=5120 takes 46 us at 64 rows there and 33 here, 62 on the
+// wave: K=5120 N=5120 takes 46 us at 64 rows there and 29 here, 61 on the
 // INT8 matrix instructions (record quantizer included).
 //
 // No barriers: a wave expands its own weights in its own LDS.  AHEAD chunks

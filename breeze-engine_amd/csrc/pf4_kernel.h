@@ -10,10 +10,11 @@ namespace bq {
 // matrix instructions (18 ns each on one SIMD) and 32 vector instructions
 // (24 ns with two waves issuing); on this GPU the two overlap little, and a
 // copy of the compute alone takes 74-85 ns a step whatever the order of its
-// instructions, 120 us at K=5120 N=17408 and 512 rows.  The kernel takes 153
-// there: operand loads (vector memory issue, 16 cycles of the CU per 1 KB
-// load) and the expansion of the weights add the rest.  On INT8 matrix
-// instructions (64 vector instructions a step) it took 196.
+// instructions, 120 us at K=5120 N=17408 and 512 rows.  The call takes 161
+// there, 5 of them the record quantizer: operand loads (vector memory issue,
+// 16 cycles of the CU per 1 KB load), the expansion of the weights and the
+// stores (4 us a round, the rate that memory takes writes at) add the rest.
+// On INT8 matrix instructions (64 vector instructions a step) it took 209.
 //
 // Split: wave (rp, part) takes 32 rows and its part of the workgroup's column
 // groups.  The rows' operands go from L2 straight to registers, reused over
@@ -134,9 +135,9 @@ __global__ __launch_bounds__((Pf4Shape<CT, RP>::kThreads)) void pf4_kernel(Pf4Ar
     };
 
     // The stage's blocks; each is reloaded a stage ahead once used.  The first
-    // loads go out before the wait for the first weights (K=5120 N=17408, 64 rows:
-    // 61.7 -> 58.1 us), but not where two runs of column
-    // groups share registers that are full: 26 spilled registers become 79 there.
+    // loads go out before the wait for the first weights (K=5120 N=17408, 64
+    // rows: 61.7 -> 58.1 us), but not where two runs of column groups share
+    // registers that are full: 26 spilled registers become 79 there.
     F6Rows<HP> ab[4];
     constexpr bool kEarlyRows = !HP || L::kGroupRem == 0;
     auto load_first = [&]() __attribute__((always_inline)) {
@@ -278,7 +279,8 @@ __global__ __launch_bounds__((Pf4Shape<CT, RP>::kThreads)) void pf4_kernel(Pf4Ar
         // Stores.  The two tiles of a group have uniform numbers, and what is
         // read of their segments stays in scalar registers: loads and stores
         // share a counter, so a vector load ahead of a store makes it wait for
-        // every store before it.
+        // every store before it (K=512 N=17408, 1024 rows: 59.0 -> 48.9 us
+        // without).
         const int m0 = rpair * 32 + 4 * kh;
         const bool odd = c32 & 16, whole = rpair * 32 + 32 <= a.M;
         auto column0 = [&](int t, int& n) __attribute__((always_inline)) {

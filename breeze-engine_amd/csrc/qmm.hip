@@ -1251,10 +1251,9 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //   paired and multi-projection calls past 32 rows  one INT4 prefill launch
 //     over all projections' tiles (two launches each, records and GEMM,
 //     before).  K=5120, with the INT8-MFMA GEMM then -> now: gate/up (N=17408)
-//     with SiLU at 33 / 200 / 512 rows 162 / 259 / 457 -> 91 / 162 / 344 (207 at
-//     200 rows as two launches of this kernel); RMSNorm + in_qkv/z/b/a at 33 /
-//     128 / 300 rows 247 / 283 / 345 -> 62 / 88 / 131; q/k/v 183 / 208 / 306 ->
-//     44 / 63 / 112.
+//     with SiLU at 33 / 200 / 512 rows 161 / 259 / 440 -> 88 / 153 / 334;
+//     RMSNorm + in_qkv/z/b/a at 33 / 128 / 256 rows 246 / 283 / 304 -> 61 / 77
+//     / 99; q/k/v (N=4096, 1024, 1024) 180 / 207 / 212 -> 30 / 47 / 59.
 //   kPf4Costs, kPf16Cost4  the rest of the INT4 prefill takes the launch of
 //     least cost: 4.9 us, then per round of workgroups 1.7 us, 60 ns a row
 //     pair by column tile (the stores) and the shape's ns a block.  Zero
@@ -1274,10 +1273,10 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //     a CU.
 //   Pf4Cost::i8  one projection past 64 rows with explicit zero points under
 //     INT8 activations compares its FP6 launch with workgroups on the INT8
-//     matrix instructions (nibble - zp in bytes): one digit there as here, and
-//     no zero-point FMA, 48 vector instructions a step on both, but the rows
-//     come through LDS and the stores and the first stage cost 2 us a round
-//     less.  FP6 -> INT8: K=5120 N=17408 at 128 / 512 rows 78.7 -> 71 / 160.6 ->
+//     matrix instructions (nibble - zp in bytes).  Both take one matrix
+//     instruction and 48 vector instructions a step (there the conversion of
+//     the integer, here the zero point's FMA), but there the rows come through
+//     LDS once a workgroup and a round costs 2 us less.  FP6 -> INT8: K=5120 N=17408 at 128 / 512 rows 78.7 -> 71 / 160.6 ->
 //     148, K=1024 N=17408 1024 rows 80.9 -> 71.4, N=5120 400 rows 22.0 ->
 //     20.3; FP6 stays where a shape fits better (K=5120 N=2560, 320 rows: 47
 //     against 61).  Over K 512 to 12288 and N 1024 to 27648 the pick is 0.5%

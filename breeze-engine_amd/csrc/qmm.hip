@@ -1232,14 +1232,21 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //   kPf16Cost8, pf8_cost  an INT8 prefill of up to 13 output tiles of 16x16 a
 //     CU (kPf16TilesPerCu) runs as independent 16-row waves (pf16_w8_kernel)
 //     where these cost less than workgroups (prefill_kernel).  A wave's time
-//     steps with the workgroups on the busiest CU, by 70 ns a block in two
-//     passes, 85 with per-block scales, 49 and 60 with INT8 activations;
-//     workgroups hardly depend on the scales.  Workgroups -> waves, K=5120:
-//     N=5120 at 33 / 64 / 128 rows 47 / 47 / 58 -> 21 / 31 / 43; kept on
-//     workgroups with per-block scales: N=17408 at 48 rows 56 (waves 64),
-//     N=10240 at 80 rows 55 (65), K=12288 N=17408 at 24 / 33 rows 104 / 127
-//     (135 / 171), K=1024 N=17408 at 33 rows 16.2 (19.2).  Past 13 tiles a CU
-//     N=5120 at 200 rows takes 60 on workgroups, 70 on waves.
+//     steps with the workgroups on the busiest CU, by 85 ns a block in two
+//     passes, 96 with per-block scales, 49 and 59 with INT8 activations, and
+//     waits longer for weights that come from memory; workgroups hardly depend
+//     on either.  Fitted with the weights read from memory (a model's other
+//     layers lie between two calls), K 512 to 12288, N 1024 to 27648, and 4%
+//     in the waves' favour (kPf16Margin8): where the two are even from memory,
+//     the waves are up to a third faster with the weights in the memory-side
+//     cache (INT8 activations, K=5120 N=10240, 64 rows: 38.8 against 39.6, 28
+//     against 38).  So picked, no call is slower than on workgroups from the
+//     cache, and 1% of them by over 3% from memory.  Workgroups -> waves,
+//     K=5120: N=5120 at 33 / 64 / 128 rows 47 / 47 / 58 -> 21 / 31 / 43; kept
+//     on workgroups: N=17408 at 17 / 48 rows 47 / 64 (waves 60 / 74), K=12288
+//     N=10240 64 rows 106 (126); with per-block scales K=5120 N=10240 80 rows
+//     55 (65), K=12288 N=17408 at 24 / 33 rows 104 / 127 (135 / 171).  Past 13
+//     tiles a CU N=5120 at 200 rows takes 60 on workgroups, 70 on waves.
 //   kPf16TilesPerCu (13), kPf16DeepPerCu (6)  the INT4 prefill runs as
 //     independent 16-row waves (pf16_kernel) up to 13 output tiles of 16x16 a
 //     CU, with four weight chunks in flight up to 6 tiles a CU and two past
@@ -1534,25 +1541,29 @@ int split_pieces(const Shape& h, int M, const CallKind& k, int n_cu, int* lds) {
 
 // What a prefill call takes by its launch, in ns (see the routing table).
 //
-// Independent 16-row waves: per workgroup of the busiest CU `start` ns and
-// `per` ns a block, besides `once` ns a block.
+// Independent 16-row waves: `call` ns, per workgroup of the busiest CU `start`
+// ns and `per` ns a block, and a block `once` ns and `read` ns a thousand
+// column tiles (weights that come from memory).
 struct Pf16Cost {
-    int start, once, per;
+    int call, start, once, per, read;
 };
-double pf16_cost(const Pf16Cost& c, int nblk, long waves, int n_cu) {
+double pf16_cost(const Pf16Cost& c, int nblk, int tiles, long waves, int n_cu) {
     const long wgs = (waves + kPf16Waves - 1) / kPf16Waves, n = (wgs + n_cu - 1) / n_cu;
-    return 4550.0 + (double)(n * c.start) + nblk * (c.once + (double)(n * c.per));
+    return c.call + (double)(n * c.start) + nblk * (c.once + (double)(n * c.per) + 0.001 * c.read * tiles);
 }
 // INT8 weights, by (two-pass, per-block scales).
-constexpr Pf16Cost kPf16Cost8[2][2] = {{{550, 5, 49}, {550, 10, 60}}, {{700, 24, 70}, {700, 20, 85}}};
+constexpr Pf16Cost kPf16Cost8[2][2] = {{{4700, 200, 31, 49, 34}, {4300, 450, 33, 59, 43}},
+                                       {{4000, 600, 26, 85, 48}, {3800, 900, 25, 96, 54}}};
+constexpr double kPf16Margin8 = 1.04;
 // Their workgroups (prefill_kernel): rounds of one a CU, `simd` tiles on the
 // busiest SIMD; a block takes a tenth less where one of four row pairs idles.
-double pf8_cost(int nblk, int rounds, int simd, bool hp, bool idle) {
-    const double ns = (hp ? 160 + 44 * simd : 155 + 28 * simd) * (idle ? 0.9 : 1.0);
-    return 4900.0 + (double)rounds * (400 * simd + nblk * ns);
+double pf8_cost(int nblk, int tiles, int rounds, int simd, bool hp, bool idle) {
+    const double ns = rounds * (hp ? 157 + 47 * simd : 85 + 54 * simd) * (idle ? 0.9 : 1.0);
+    return 5000.0 + nblk * (ns + 0.001 * (hp ? 11 : 3) * tiles);
 }
 // INT4, by (explicit zero points, four weight chunks in flight).
-constexpr Pf16Cost kPf16Cost4[2][2] = {{{550, 97, 57}, {550, 76, 47}}, {{800, 66, 80}, {800, 58, 74}}};
+constexpr Pf16Cost kPf16Cost4[2][2] = {{{4550, 550, 97, 57, 0}, {4550, 550, 76, 47, 0}},
+                                       {{4550, 800, 66, 80, 0}, {4550, 800, 58, 74, 0}}};
 // INT4 workgroup shapes: ns a block of one round, for two-pass calls, two-pass with
 // zero points, INT8 activations, and those with zero points.  Shapes of four
 // waves run two workgroups a CU; `half` is for a single round of one.  `i8`:
@@ -1642,7 +1653,7 @@ bool pick_pf16(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, int
                 !std::getenv("BREEZE_HIP_PREFILL_CT");
     if (take && !(h.bits == 4 && pf4_plain(h, k))) {
         const Pf16Cost& c = h.bits == 8 ? kPf16Cost8[k.hp][h.extra] : kPf16Cost4[h.has_zp][deep];
-        take = pf16_cost(c, h.nblk, waves, n_cu) <= wg_cost;
+        take = pf16_cost(c, h.nblk, tiles, waves, n_cu) <= wg_cost * (h.bits == 8 ? kPf16Margin8 : 1.0);
     }
     if (!(env ? env[0] == '1' : take)) return false;
     p.pf_rp = 0;
@@ -1746,7 +1757,7 @@ Plan plan_call(const Shape& h, int M, const CallKind& k, int n_cu) {
             return p;
         }
         const bool idle = p.grid_y == 1 && p.pf_rp == 4 && M <= 96;
-        if (pick_pf16(p, h, k, M, tiles, n_cu, pf8_cost(h.nblk, rounds, simd, k.hp, idle))) return p;
+        if (pick_pf16(p, h, k, M, tiles, n_cu, pf8_cost(h.nblk, tiles, rounds, simd, k.hp, idle))) return p;
         p.pf_ct = ct;
         p.grid_x = (tiles + p.pf_ct - 1) / p.pf_ct;
     } else if (dec8) {

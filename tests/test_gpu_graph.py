@@ -93,7 +93,7 @@ def test_captured_argmax_replays_exact(gpu, hb, hi_prec):
     ((8, 128), (4, 128)),   # INT8 weights, then INT4 (FP6 records)
     ((4, 128), (8, 128)),
 ])
-def test_capture_after_a_call_of_as_many_rows(gpu, hb, orc, hi_prec, first, then):
+def test_capture_after_a_call_of_as_many_rows(gpu, hb, orc, hi_prec, monkeypatch, first, then):
     """A stream's room for the prefill's records depends on the rows and K
     alone, so after one call a call of no more rows is captured without an
     allocation, whatever its launch and weights; replays are bit-exact with
@@ -108,17 +108,24 @@ def test_capture_after_a_call_of_as_many_rows(gpu, hb, orc, hi_prec, first, then
         weights[bits] = (qw, sc)
         handles[bits] = hb.prepack(qw, sc, None, K, N, bits=bits)
     hb.set_hi_prec(True)
-    if first[0] == then[0] == 8:
-        assert hb.plan(8, first[1], K, N)["pf_rp"] == 4 and hb.plan(8, then[1], K, N)["pf_rp"] == 0
+    waves = first[0] == then[0] == 8
+
+    def launch(which):
+        if waves:
+            monkeypatch.setenv("BREEZE_HIP_PF16", "01"[which == then])
+            assert (hb.plan(8, which[1], K, N)["pf_rp"] == 0) == (which == then)
+
     try:
         cap = torch.cuda.Stream()
         a0 = torch.from_numpy(rng.normal(size=(first[1], K)).astype(np.float32)).cuda()
         A = [rng.normal(size=(then[1], K)).astype(np.float32) for _ in range(3)]
         x = torch.from_numpy(A[0]).cuda()
         torch.cuda.synchronize()
+        launch(first)
         with torch.cuda.stream(cap):
             hb.matmul(handles[first[0]], a0, N)
         torch.cuda.synchronize()
+        launch(then)
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=cap):
             y = hb.matmul(handles[then[0]], x, N)

@@ -1,6 +1,6 @@
 """Which launch a prefill call takes (pick_pf16, pick_pf4 in csrc/qmm.hip): few
 output tiles a CU go to independent 16-row waves (pf_rp 0), more to a
-workgroup shape, for INT4 the one with the fewest rounds of column groups."""
+workgroup shape, for INT4 the one of least cost (kPf4Costs)."""
 import pytest
 
 TABLE = [

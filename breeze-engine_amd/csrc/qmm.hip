@@ -1236,13 +1236,15 @@ void fill_args(const Handle* h, GemvArgs& a, int M) {
 //     passes, 96 with per-block scales, 49 and 59 with INT8 activations, and
 //     waits longer for weights that come from memory; workgroups hardly depend
 //     on either.  Fitted with the weights read from memory (a model's other
-//     layers lie between two calls), K 512 to 12288, N 1024 to 27648, and 4%
-//     in the waves' favour (kPf16Margin8): where the two are even from memory,
-//     the waves are up to a third faster with the weights in the memory-side
-//     cache (INT8 activations, K=5120 N=10240, 64 rows: 38.8 against 39.6, 28
-//     against 38).  So picked, no call is slower than on workgroups from the
-//     cache, and 1% of them by over 3% from memory.  Workgroups -> waves,
-//     K=5120: N=5120 at 33 / 64 / 128 rows 47 / 47 / 58 -> 21 / 31 / 43; kept
+//     layers lie between two calls), K 512 to 12288, N 1024 to 27648, and 7%
+//     in the waves' favour, 4 with per-block scales (kPf16Margin8): where the
+//     two are even from memory, the waves are up to a third faster with the
+//     weights in the memory-side cache (INT8 activations, K=5120 N=10240, 64
+//     rows: 38.8 against 39.6, 28 against 38).  At 4% for both, waves that are
+//     faster either way stayed on workgroups (INT8 activations, K=1024
+//     N=12288, 33 rows: 11.9 against 12.6, 10.4 against 12.4).  So picked, no
+//     call is slower than on workgroups from the cache, and 1% of them by over
+//     3% from memory.  Workgroups -> waves, K=5120: N=5120 at 33 / 64 / 128 rows 47 / 47 / 58 -> 21 / 31 / 43; kept
 //     on workgroups: N=17408 at 17 / 48 rows 47 / 64 (waves 60 / 74), K=12288
 //     N=10240 64 rows 106 (126); with per-block scales K=5120 N=10240 80 rows
 //     55 (65), K=12288 N=17408 at 24 / 33 rows 104 / 127 (135 / 171).  Past 13
@@ -1554,7 +1556,7 @@ double pf16_cost(const Pf16Cost& c, int nblk, int tiles, long waves, int n_cu) {
 // INT8 weights, by (two-pass, per-block scales).
 constexpr Pf16Cost kPf16Cost8[2][2] = {{{4700, 200, 31, 49, 34}, {4300, 450, 33, 59, 43}},
                                        {{4000, 600, 26, 85, 48}, {3800, 900, 25, 96, 54}}};
-constexpr double kPf16Margin8 = 1.04;
+constexpr double kPf16Margin8[2] = {1.07, 1.04};  // by per-block scales
 // Their workgroups (prefill_kernel): rounds of one a CU, `simd` tiles on the
 // busiest SIMD; a block takes a tenth less where one of four row pairs idles.
 double pf8_cost(int nblk, int tiles, int rounds, int simd, bool hp, bool idle) {
@@ -1653,7 +1655,7 @@ bool pick_pf16(Plan& p, const Shape& h, const CallKind& k, int M, int tiles, int
                 !std::getenv("BREEZE_HIP_PREFILL_CT");
     if (take && !(h.bits == 4 && pf4_plain(h, k))) {
         const Pf16Cost& c = h.bits == 8 ? kPf16Cost8[k.hp][h.extra] : kPf16Cost4[h.has_zp][deep];
-        take = pf16_cost(c, h.nblk, tiles, waves, n_cu) <= wg_cost * (h.bits == 8 ? kPf16Margin8 : 1.0);
+        take = pf16_cost(c, h.nblk, tiles, waves, n_cu) <= wg_cost * (h.bits == 8 ? kPf16Margin8[h.extra] : 1.0);
     }
     if (!(env ? env[0] == '1' : take)) return false;
     p.pf_rp = 0;

@@ -50,6 +50,17 @@ def test_int8_prefill_launch(hb, shape, want):
     assert {k: got[k] for k in want} == want, got
 
 
+def test_int8_waves_that_are_faster_either_way(hb):
+    """INT8 activations, K=1024 N=12288, 33 rows: waves 10.4 us with the weights
+    in the memory-side cache and 11.9 from memory, workgroups 12.4 and 12.6;
+    K=2048: 14.6 and 18.1, 19.1 and 19.5.  K=5120 N=12288 with per-block scales,
+    where the waves lose 15% from memory, stays on workgroups."""
+    for K in (1024, 2048):
+        for M in (33, 48, 64):
+            assert hb.plan(8, M, K, 12288, hi=False)["pf_rp"] == 0
+    assert hb.plan(8, 33, 5120, 12288, hi=False, extra=True)["pf_rp"] == 2
+
+
 def test_projections_share_a_prefill_launch(hb):
     """Past 32 rows the gate/up pair (twice the tiles) and multi-projection
     calls take one INT4 prefill launch; INT8 ones, the fused norm, argmax and
